@@ -242,7 +242,9 @@ typedef struct mcd_launch {
  * through LDS, so the transport code carries no FP64; for mcd_batch_run the
  * block may then be 128 to 1024).  Records are identical in every form.
  * Without a flag (and without block or waves_per_simd), mcd_forward runs DS
- * launches of at least 2^21 electrons served and smaller ones inline;
+ * launches of at least 2^21 electrons served and smaller ones inline; those too
+ * small to fill the GPU with one lane per electron (up to 384 electrons per
+ * CU) run with 4 to 64 lanes per electron, guard inline;
  * mcd_batch_run runs inline unless another form is asked for (the faster form
  * depends on the configuration; mcd/autotune.py measures it).  Setting more
  * than one flag is an error. */
@@ -371,7 +373,8 @@ int mcd_forward(mcd_ctx* ctx, const mcd_config* cfg, const mcd_tables* tables, u
 /* mcd_forward that allocates nothing: no reference counterpart; for callers
  * that cannot allocate device memory (code under HIP graph capture, serving
  * loops, harnesses that forbid hipMalloc).  Same arguments, records and
- * counters as mcd_forward.  A DS FP32 launch runs the deferred guard unless a
+ * counters as mcd_forward.  A DS FP32 launch too large for several lanes per
+ * electron (see above) runs the deferred guard unless a
  * guard flag asks for another form, and parks its electrons in the library's
  * static device scratch (MCD_NOALLOC_MAX_ELECTRONS park records, ~72 MiB held
  * by each GPU the library runs on until the process ends); every other launch

@@ -1100,7 +1100,13 @@ static int forward_impl(mcd_ctx* ctx, const mcd_config* cfg, const mcd_tables* t
     return set_err(ctx, MCD_ERR_INVALID, service ? "service guard: waves_per_simd %d not 6, 7 or 8"
                                                  : "waves_per_simd %d not one of 1, 4, 5, 6, 8", minw);
   const uint64_t want = (n + block - 1) / block;
-  if (service) {
+  // launches too small to fill the chip with one lane per electron take
+  // several lanes per electron, unless a placement or a shape is asked for
+  const int wlg = ds32 && !guard_flags && !shape_given && !R.rows ? window_log2_lanes(c, n, ctx->n_cu) : 0;
+  if (wlg) {
+    HIP_TRY(ctx, launch_fill_u64(q, 0ull, 1, s));
+    HIP_TRY(ctx, launch_window_ds(c, R, wlg, s));
+  } else if (service) {
     // wavefront 0 of each workgroup serves the guard; the others carry electrons
     const uint64_t want_svc = (n + (uint64_t)(block - 64) - 1) / (uint64_t)(block - 64);
     uint64_t grid = (uint64_t)ctx->n_cu * (uint64_t)svc_blocks_per_cu(c, minw, block);

@@ -11,93 +11,9 @@
 
 #include "mcd_device.h"
 #include "mcd_internal.h"
+#include "mcd_step.h"
 
 namespace mcd {
-
-// LDS of the one-configuration kernels: the pick table (nf floats), then the
-// two loss-table descriptors at a 16-byte aligned offset.
-__host__ __device__ constexpr int tab_offset_floats(int nf) { return (nf + 3) & ~3; }
-static size_t single_lds_bytes(const DevCfg& c) {
-  return (size_t)tab_offset_floats(c.pick.n_nodes * c.pick.stride) * sizeof(float) + 2 * sizeof(DevTable);
-}
-
-// Stage the pick table and the two loss-table descriptors (Moller,
-// Gryzinski) that a lane selects by its channel.
-__device__ __forceinline__ DevTable* stage_single(const DevCfg& c, float* lds) {
-  const int nf = c.pick.n_nodes * c.pick.stride;
-  for (int i = threadIdx.x; i < nf; i += blockDim.x) lds[i] = c.pick.nodes[i];
-  DevTable* tabs = reinterpret_cast<DevTable*>(lds + tab_offset_floats(nf));
-  if (threadIdx.x == 0) {
-    tabs[0] = c.tm;
-    tabs[1] = c.tg;
-  }
-  return tabs;
-}
-
-// The served kernel's LDS copy of the pick table in the wide record
-// (pick_stride_wide): each node's record, then its differences to the next
-// node, each the same float subtraction the compact record's interpolation
-// does at every step, so the interpolated values are the same bit for bit.
-template <int NCH>
-__device__ __forceinline__ DevTable* stage_single_wide(const DevCfg& c, float* lds) {
-  constexpr int S = pick_stride(NCH), SW = pick_stride_wide(NCH), NB = NCH - 1, D = NB + 3;
-  const int n = c.pick.n_nodes;
-  const float* __restrict__ g = c.pick.nodes;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const float* a = g + (size_t)k * S;
-    float* o = lds + (size_t)k * SW;
-    for (int i = 0; i < D; ++i) o[i] = a[i];
-    for (int i = 0; i <= NB; ++i) o[D + i] = k + 1 < n ? a[S + i] - a[i] : 0.f;
-  }
-  DevTable* tabs = reinterpret_cast<DevTable*>(lds + tab_offset_floats(n * SW));
-  if (threadIdx.x == 0) {
-    tabs[0] = c.tm;
-    tabs[1] = c.tg;
-  }
-  return tabs;
-}
-
-// The record is written once, when the trajectory ends, as nine dword
-// stores marked non-temporal: records of one wavefront land in different
-// cache lines at different times, and streaming them past L2 keeps them from
-// evicting the loss tables and from being read back to merge partial lines.
-__device__ __forceinline__ void write_rec(mcd_electron_rec* rec, float E, const float* d, const float* p, uint32_t nsc,
-                                          int o1, int o2, uint32_t flags) {
-  uint32_t* w = reinterpret_cast<uint32_t*>(rec);
-  __builtin_nontemporal_store(__float_as_uint(E), w + 0);
-  __builtin_nontemporal_store(__float_as_uint(d[0]), w + 1);
-  __builtin_nontemporal_store(__float_as_uint(d[1]), w + 2);
-  __builtin_nontemporal_store(__float_as_uint(d[2]), w + 3);
-  __builtin_nontemporal_store(__float_as_uint(p[0]), w + 4);
-  __builtin_nontemporal_store(__float_as_uint(p[1]), w + 5);
-  __builtin_nontemporal_store(__float_as_uint(p[2]), w + 6);
-  __builtin_nontemporal_store(nsc, w + 7);
-  // outcome, outcome2, flags, pad (bytes 32..35, little endian)
-  __builtin_nontemporal_store((uint32_t)(o1 & 0xFF) | ((uint32_t)(o2 & 0xFF) << 8) | ((flags & 0xFFu) << 16), w + 8);
-}
-
-// wave-level append of scatter rows; returns the slot or ~0 when full
-__device__ __forceinline__ uint64_t append_slot(bool want, unsigned long long* cursor, uint64_t cap, int lane) {
-  uint64_t m = __ballot(want);
-  if (!m) return ~0ull;
-  int leader = __ffsll((unsigned long long)m) - 1;
-  unsigned long long base = 0;
-  if (lane == leader) base = atomicAdd(cursor, (unsigned long long)__popcll(m));
-  base = lane_u64(base, leader);
-  uint64_t slot = base + __popcll(m & ((1ull << lane) - 1ull));
-  return (want && slot < cap) ? slot : ~0ull;
-}
-
-__device__ __forceinline__ void wave_add_counters(unsigned long long* cnt, const uint64_t* v, int nv, int lane) {
-  for (int i = 0; i < nv; ++i) {
-    uint64_t x = v[i];
-    for (int off = 32; off > 0; off >>= 1) {
-      uint32_t lo = __shfl_xor((uint32_t)x, off), hi = __shfl_xor((uint32_t)(x >> 32), off);
-      x += ((uint64_t)hi << 32) | lo;
-    }
-    if (lane == 0 && x) atomicAdd(&cnt[i], (unsigned long long)x);
-  }
-}
 
 // Counts of records i0, i0 + step, ... < n: each thread reads only the
 // records' outcome dword (byte 32: outcome, outcome2, flags), the wavefronts
@@ -163,23 +79,6 @@ __device__ __forceinline__ uint32_t box_load(const uint32_t* p) {
 }
 __device__ __forceinline__ void box_store(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-// The channel order d_pick_ordered expects: a crossing cell's swap was
-// applied to pe.perm by the interpolation; undo it so the FP64 pick sees node
-// k's order and decides the pair exactly.
-template <int NCH>
-__device__ __forceinline__ void guard_perm(const PickEval<NCH>& pe, uint32_t& plo, uint32_t& phi) {
-  plo = pe.perm_lo;
-  phi = pe.perm_hi;
-  if (pe.swap != (int)kMetaNoSwap && pe.pB > pe.pA) {
-    uint64_t pm = ((uint64_t)phi << 32) | plo;
-    const uint64_t la = (pm >> (4 * pe.swap)) & 15u, lb = (pm >> (4 * (pe.swap + 1))) & 15u;
-    pm &= ~((uint64_t)0xFFu << (4 * pe.swap));
-    pm |= (lb << (4 * pe.swap)) | (la << (4 * (pe.swap + 1)));
-    plo = (uint32_t)pm;
-    phi = (uint32_t)(pm >> 32);
-  }
 }
 
 // The service wavefront's loop: answer posted mailboxes until every transport
@@ -392,40 +291,7 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
         }
       }
       l = -mfp_ln2 * log2_f(u1);
-      // 1/E for both the screening parameter and the loss fraction: one
-      // reciprocal for the wavefront instead of one in each channel branch
-      const float rE = __builtin_amdgcn_rcpf(E.hi);
-      if (ch == MCD_CH_RUTH) {  // Rutherford_halfPol, scattering.py:125-152
-        Wh = 0.f;
-        const float a = c.c_alpha_f * rE;
-        const float om = 1.f - u2;
-        const float inv = __builtin_amdgcn_rcpf(om + a);
-        s2 = a * u2 * inv;
-        c2 = om * (1.f + a) * inv;
-      } else if (ch == MCD_CH_QUINN) {  // scattering.py:643-656
-        Wh = c.Epl_hi; Wl = c.Epl_lo;
-        c2 = 1.f; s2 = 0.f;
-      } else {  // Moller table, or the outer-shell Gryzinski table for all shells (:602-640)
-        const DevTable& t = tabs[ch == MCD_CH_MOLLER ? 0 : 1];  // LDS: no per-lane kernel-argument loads
-        const F2 Ec = E;
-        int row;
-        const int col = table_lookup(t, E.hi, [Ec](float v) { return f_lt_f2(v, Ec); }, u2, row);
-        Wh = ldg(t.Ws + col);
-        if (!f_lt_f2(Wh, E)) sflags |= MCD_FLAG_LOSS_GE_E;
-        // binaryCollModel (:156-179): W <= (E - E_F)/2
-        const F2 D = f2_sub(E, c.Ef2_hi, c.Ef2_lo);
-        const float w2 = 2.f * Wh;
-        const bool ok = !(D.hi < w2 || (D.hi == w2 && D.lo < 0.f));
-        if (ok) {
-          const float x = Wh * rE;
-          const float sq = __builtin_amdgcn_sqrtf(1.f - x);
-          c2 = 0.5f * (1.f + sq);
-          s2 = 0.5f * x * __builtin_amdgcn_rcpf(1.f + sq);
-        } else {
-          c2 = s2 = __builtin_nanf("");
-          sflags |= MCD_FLAG_NAN_DIR;
-        }
-      }
+      ds_loss_angles(c, tabs, E, ch, u2, Wh, Wl, c2, s2, sflags);
     } else {
       const float u0 = u01f(r.x), u1 = u01f(r.y);
       u_az = u01f(r.z);

@@ -231,7 +231,8 @@ class Transport:
                precision=_abi.PREC_FP32, block=0, waves_per_simd=0, guard=None, stream=None, refill_period=0):
         """Asynchronous launch on `stream` into caller-owned torch buffers.
         guard: None (library default: served for DS launches of at least 2^21
-        electrons with no shape given, inline otherwise), "inline", "deferred"
+        electrons with no shape given, inline otherwise, small ones with
+        several lanes per electron), "inline", "deferred"
         or "service" -- where the DS FP64 guard pick runs (same records in
         every form).  refill_period: the compaction period, idle lanes take
         new electrons every refill_period steps (0: every step)."""

@@ -1,0 +1,64 @@
+"""Launches with several lanes per electron (mcd_window.hip) against one lane
+per electron: the same formulas step by step, so records, scatter rows and
+counters are equal bit for bit."""
+import numpy as np
+import pytest
+
+from mcd import _abi, engine
+
+pytestmark = pytest.mark.gpu
+
+COUNTED = [_abi.CNT_EVENTS, _abi.CNT_ELECTRONS, _abi.CNT_BKS, _abi.CNT_ABS, _abi.CNT_TRSM, _abi.CNT_LONG,
+           _abi.CNT_FP64_PICKS, _abi.CNT_SCAT_ROWS, _abi.CNT_GUARD_TIMEOUTS]
+INF = float("inf")
+
+
+def _transport(material="Cu", E0=20000.0, Emin=1000.0, Wc=50.0, tilt=70.0, **kw):
+    return engine.Transport(material, E0, Emin, Wc=Wc, s_tilt=tilt, tol_E=1e-2, tol_W=1e-2, grid_search="library", **kw)
+
+
+def _same(a, b):
+    assert a.els.tobytes() == b.els.tobytes()
+    assert np.array_equal(a.counters[COUNTED], b.counters[COUNTED])
+    if b.scats is not None:
+        assert a.scats.tobytes() == b.scats.tobytes()
+
+
+@pytest.fixture(scope="module")
+def cu():
+    return _transport()
+
+
+# the counts around which the lanes per electron change (256 CUs: 3840 << 6 =
+# 7680 << 5 = .. = 98304 * 2.5), one electron, one short of and past a wavefront
+@pytest.mark.parametrize("n", [1, 3, 63, 65, 3840, 3841, 7680, 7681, 15361, 30720, 30721, 98304, 98305])
+def test_ds_sizes_equal_one_lane_per_electron(cu, n):
+    _same(cu.run(n, seed=n), cu.run(n, seed=n, guard="inline"))
+
+
+@pytest.mark.parametrize("kw", [
+    dict(material="Al", E0=5000.0, Emin=500.0, tilt=0.0),
+    dict(material="Si", E0=1600.0, Wc=10.0, tilt=85.0),
+    dict(material="Au", E0=30000.0, Wc=20.0, elastic="Ruth_nigram"),
+    dict(material="Au", E0=5000.0, Emin=500.0, tilt=0.0, thickness=2000.0),
+    dict(max_scatt=1), dict(max_scatt=63), dict(max_scatt=64), dict(max_scatt=65, thickness=20000.0, tilt=0.0),
+], ids=str)
+@pytest.mark.parametrize("n,first", [(5, (1 << 32) - 3), (700, 0), (20001, 17)])
+def test_ds_configurations_equal_one_lane_per_electron(kw, n, first):
+    tr = _transport(**kw)
+    _same(tr.run(n, seed=4, first=first), tr.run(n, seed=4, first=first, guard="inline"))
+
+
+@pytest.mark.parametrize("n,kept", [(1, 1), (70, 70), (300, 33)])
+@pytest.mark.parametrize("kw", [dict(), dict(max_scatt=65), dict(material="Si", E0=10000.0, tilt=0.0, thickness=3000.0)],
+                         ids=str)
+def test_ds_scatter_rows_equal_one_lane_per_electron(kw, n, kept):
+    tr = _transport(**kw)
+    a = tr.run(n, seed=9, first=5, scats=True, scat_max_electron=5 + kept)
+    _same(a, tr.run(n, seed=9, first=5, scats=True, scat_max_electron=5 + kept, guard="inline"))
+
+
+def test_repeated_runs_are_equal(cu):
+    a = cu.run(12345, seed=8)
+    for _ in range(3):
+        _same(cu.run(12345, seed=8), a)
