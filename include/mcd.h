@@ -427,6 +427,19 @@ int mcd_batch_destroy(mcd_batch* b);
 int mcd_scatter_pack(mcd_ctx* ctx, const mcd_scatter_rec* rows, uint64_t n_rows, uint32_t fields, void* out,
                      size_t out_bytes, size_t* needed, void* stream);
 
+/* The scatter rows of one launch in (electron, step) order, with the selected
+ * fields (a mask of MCD_SCAT_*; all of them: whole mcd_scatter_rec) of each row
+ * next to each other in record order, no padding.  rows: the n_rows rows of a
+ * launch that did not overflow; els: the launch's records of the n_els
+ * electrons [first, first + n_els) that recorded rows (a row's place follows
+ * from the scatter counts of the electrons before it, so nothing is compared or
+ * sorted).  *needed receives the bytes out must hold: the packed rows, then at
+ * the next multiple of 256 bytes scratch of 8 bytes per electron; out = NULL
+ * asks for that size only.  Asynchronous on stream. */
+int mcd_scatter_rows(mcd_ctx* ctx, const mcd_scatter_rec* rows, uint64_t n_rows, const mcd_electron_rec* els,
+                     uint64_t n_els, uint64_t first, uint32_t fields, void* out, size_t out_bytes, size_t* needed,
+                     void* stream);
+
 /* Differentiation (no reference counterpart).  Derivatives of
  *   Y   = number of backscattered electrons (outcome 'bks', electron.py:68-70)
  *   H_b = number of backscattered electrons whose exit energy (the pre-step

@@ -1102,7 +1102,7 @@ static int forward_impl(mcd_ctx* ctx, const mcd_config* cfg, const mcd_tables* t
   const uint64_t want = (n + block - 1) / block;
   // launches too small to fill the chip with one lane per electron take
   // several lanes per electron, unless a placement or a shape is asked for
-  const int wlg = ds32 && !guard_flags && !shape_given && !R.rows ? window_log2_lanes(c, n, ctx->n_cu) : 0;
+  const int wlg = ds32 && !guard_flags && !shape_given ? window_log2_lanes(c, n, ctx->n_cu) : 0;
   if (wlg) {
     HIP_TRY(ctx, launch_fill_u64(q, 0ull, 1, s));
     HIP_TRY(ctx, launch_window_ds(c, R, wlg, s));
@@ -1442,33 +1442,36 @@ extern "C" int mcd_batch_run(mcd_ctx* ctx, mcd_batch* b, uint64_t seed, uint64_t
 }
 
 // ---------------------------------------------------------------------------
+// Offsets and sizes of mcd_scatter_rec's fields, in record order.
+typedef mcd_scatter_rec ScatRec;
+static const int kScatOff[kScatFields] = {
+    (int)offsetof(ScatRec, electron), (int)offsetof(ScatRec, step), (int)offsetof(ScatRec, config),
+    (int)offsetof(ScatRec, channel), (int)offsetof(ScatRec, outcome), (int)offsetof(ScatRec, E),
+    (int)offsetof(ScatRec, E_loss), (int)offsetof(ScatRec, pol), (int)offsetof(ScatRec, az),
+    (int)offsetof(ScatRec, pathl), (int)offsetof(ScatRec, x), (int)offsetof(ScatRec, y), (int)offsetof(ScatRec, z),
+    (int)offsetof(ScatRec, energy), (int)offsetof(ScatRec, dx), (int)offsetof(ScatRec, dy),
+    (int)offsetof(ScatRec, dz), (int)offsetof(ScatRec, step_flags)};
+static const int kScatSize[kScatFields] = {
+    (int)sizeof(ScatRec::electron), (int)sizeof(ScatRec::step), (int)sizeof(ScatRec::config),
+    (int)sizeof(ScatRec::channel), (int)sizeof(ScatRec::outcome), (int)sizeof(ScatRec::E),
+    (int)sizeof(ScatRec::E_loss), (int)sizeof(ScatRec::pol), (int)sizeof(ScatRec::az), (int)sizeof(ScatRec::pathl),
+    (int)sizeof(ScatRec::x), (int)sizeof(ScatRec::y), (int)sizeof(ScatRec::z), (int)sizeof(ScatRec::energy),
+    (int)sizeof(ScatRec::dx), (int)sizeof(ScatRec::dy), (int)sizeof(ScatRec::dz), (int)sizeof(ScatRec::step_flags)};
+
 // Scatter rows to columns on the device.
 extern "C" int mcd_scatter_pack(mcd_ctx* ctx, const mcd_scatter_rec* rows, uint64_t n_rows, uint32_t fields,
                                 void* out, size_t out_bytes, size_t* needed, void* stream) {
   if (!ctx || !needed) return set_err(ctx, MCD_ERR_INVALID, "mcd_scatter_pack: NULL argument");
   if (fields == 0u || (fields >> kScatFields) != 0u)
     return set_err(ctx, MCD_ERR_INVALID, "field mask 0x%x selects no field or an unknown one", fields);
-  typedef mcd_scatter_rec R;
-  static const int off[kScatFields] = {
-      (int)offsetof(R, electron), (int)offsetof(R, step), (int)offsetof(R, config), (int)offsetof(R, channel),
-      (int)offsetof(R, outcome), (int)offsetof(R, E), (int)offsetof(R, E_loss), (int)offsetof(R, pol),
-      (int)offsetof(R, az), (int)offsetof(R, pathl), (int)offsetof(R, x), (int)offsetof(R, y),
-      (int)offsetof(R, z), (int)offsetof(R, energy), (int)offsetof(R, dx), (int)offsetof(R, dy),
-      (int)offsetof(R, dz), (int)offsetof(R, step_flags)};
-  static const int sz[kScatFields] = {
-      (int)sizeof(R::electron), (int)sizeof(R::step), (int)sizeof(R::config), (int)sizeof(R::channel),
-      (int)sizeof(R::outcome), (int)sizeof(R::E), (int)sizeof(R::E_loss), (int)sizeof(R::pol),
-      (int)sizeof(R::az), (int)sizeof(R::pathl), (int)sizeof(R::x), (int)sizeof(R::y),
-      (int)sizeof(R::z), (int)sizeof(R::energy), (int)sizeof(R::dx), (int)sizeof(R::dy),
-      (int)sizeof(R::dz), (int)sizeof(R::step_flags)};
   ScatPackPlan plan{};
   uint64_t at = 0;
   for (int f = 0; f < kScatFields; ++f) {
     if (!((fields >> f) & 1u)) continue;
-    plan.src[plan.n] = off[f];
-    plan.size[plan.n] = sz[f];
+    plan.src[plan.n] = kScatOff[f];
+    plan.size[plan.n] = kScatSize[f];
     plan.dst[plan.n] = at;
-    at += (n_rows * (uint64_t)sz[f] + 255u) / 256u * 256u;
+    at += (n_rows * (uint64_t)kScatSize[f] + 255u) / 256u * 256u;
     plan.n++;
   }
   *needed = (size_t)at;
@@ -1479,6 +1482,38 @@ extern "C" int mcd_scatter_pack(mcd_ctx* ctx, const mcd_scatter_rec* rows, uint6
                    (unsigned long long)at);
   HIP_TRY(ctx, hipSetDevice(ctx->device));
   HIP_TRY(ctx, launch_pack_scatter(rows, n_rows, plan, out, (hipStream_t)stream));
+  return MCD_OK;
+}
+
+// Scatter rows in (electron, step) order on the device.
+extern "C" int mcd_scatter_rows(mcd_ctx* ctx, const mcd_scatter_rec* rows, uint64_t n_rows,
+                                const mcd_electron_rec* els, uint64_t n_els, uint64_t first, uint32_t fields,
+                                void* out, size_t out_bytes, size_t* needed, void* stream) {
+  if (!ctx || !needed) return set_err(ctx, MCD_ERR_INVALID, "mcd_scatter_rows: NULL argument");
+  if (fields == 0u || (fields >> kScatFields) != 0u)
+    return set_err(ctx, MCD_ERR_INVALID, "field mask 0x%x selects no field or an unknown one", fields);
+  if (n_els > (1ull << 32) || n_rows > (1ull << 40))
+    return set_err(ctx, MCD_ERR_INVALID, "mcd_scatter_rows: a row names its electron by 32 bits");
+  ScatPackPlan plan{};
+  int at = 0;
+  for (int f = 0; f < kScatFields; ++f) {
+    if (!((fields >> f) & 1u)) continue;
+    plan.src[plan.n] = kScatOff[f];
+    plan.size[plan.n] = kScatSize[f];
+    plan.dst[plan.n] = (uint64_t)at;
+    at += kScatSize[f];
+    plan.n++;
+  }
+  const uint64_t packed = (n_rows * (uint64_t)at + 255u) / 256u * 256u;
+  *needed = (size_t)(packed + n_els * sizeof(uint64_t));
+  if (!out) return MCD_OK;
+  if ((n_rows && !rows) || (n_els && !els)) return set_err(ctx, MCD_ERR_INVALID, "mcd_scatter_rows: NULL rows or els");
+  if (out_bytes < *needed)
+    return set_err(ctx, MCD_ERR_INVALID, "output holds %zu bytes, the rows and scratch need %zu", out_bytes, *needed);
+  HIP_TRY(ctx, hipSetDevice(ctx->device));
+  HIP_TRY(ctx, launch_order_scatter(rows, n_rows, els, n_els, (uint32_t)first, plan, at, out,
+                                    reinterpret_cast<uint64_t*>(static_cast<char*>(out) + packed),
+                                    (hipStream_t)stream));
   return MCD_OK;
 }
 

@@ -120,6 +120,12 @@ struct ScatPackPlan {
 hipError_t launch_pack_scatter(const mcd_scatter_rec* rows, uint64_t n, const ScatPackPlan& plan, void* out,
                                hipStream_t s);
 
+// Rows in (electron, step) order, the plan's fields of each side by side in
+// row_bytes (plan.dst: offsets in the packed row); starts: scratch, n_els.
+hipError_t launch_order_scatter(const mcd_scatter_rec* rows, uint64_t n, const mcd_electron_rec* els, uint64_t n_els,
+                                uint32_t first, const ScatPackPlan& plan, int row_bytes, void* out, uint64_t* starts,
+                                hipStream_t s);
+
 // tables
 hipError_t launch_build_cdf(const float* Es, const float* Ws, int nE, int nW, double Ef, int kind, double n_el,
                             double Eb, int precision, float* cdf, hipStream_t s);

@@ -949,6 +949,70 @@ hipError_t launch_pack_scatter(const mcd_scatter_rec* rows, uint64_t n, const Sc
   return hipGetLastError();
 }
 
+// First row of each electron in (electron, step) order: the exclusive prefix
+// sum of the records' scatter counts (an electron has one row per event).  One
+// workgroup: each thread adds a run of records, the workgroup scans its runs.
+__global__ __launch_bounds__(1024) void k_row_starts(const mcd_electron_rec* __restrict__ els, uint64_t n,
+                                                     uint64_t* __restrict__ starts) {
+  __shared__ uint64_t part[1024];
+  const uint64_t run = (n + blockDim.x - 1) / blockDim.x;
+  const uint64_t a = run * threadIdx.x, b = a + run < n ? a + run : n;
+  uint64_t sum = 0;
+  for (uint64_t i = a; i < b; ++i) sum += els[i].n_scatt;
+  part[threadIdx.x] = sum;
+  __syncthreads();
+  for (unsigned off = 1; off < blockDim.x; off <<= 1) {
+    const uint64_t v = threadIdx.x >= off ? part[threadIdx.x - off] : 0;
+    __syncthreads();
+    part[threadIdx.x] += v;
+    __syncthreads();
+  }
+  uint64_t at = part[threadIdx.x] - sum;
+  for (uint64_t i = a; i < b; ++i) {
+    starts[i] = at;
+    at += els[i].n_scatt;
+  }
+}
+
+// Each row to its place in (electron, step) order.  One thread per row; the
+// rows a wavefront appended lie side by side, mostly steps of one electron.
+// Bound by the 64 bytes read and the packed bytes written per row.
+__global__ __launch_bounds__(256) void k_order_scatter(const mcd_scatter_rec* __restrict__ rows, uint64_t n,
+                                                       uint64_t n_els, uint32_t first, ScatPackPlan plan,
+                                                       int row_bytes, const uint64_t* __restrict__ starts,
+                                                       uint8_t* __restrict__ out) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    const mcd_scatter_rec* r = rows + i;
+    const uint32_t el = r->electron - first;
+    if (el >= n_els) continue;
+    const uint64_t place = starts[el] + r->step;
+    if (place >= n) continue;
+    uint8_t* dst = out + place * (uint64_t)row_bytes;
+    const uint8_t* src = reinterpret_cast<const uint8_t*>(r);
+    for (int f = 0; f < plan.n; ++f) {
+      const uint8_t* v = src + plan.src[f];
+      uint8_t* w = dst + plan.dst[f];  // packed rows: any alignment
+      if (plan.size[f] == 4) __builtin_memcpy(w, v, 4);
+      else if (plan.size[f] == 2) __builtin_memcpy(w, v, 2);
+      else *w = *v;
+    }
+  }
+}
+
+hipError_t launch_order_scatter(const mcd_scatter_rec* rows, uint64_t n, const mcd_electron_rec* els, uint64_t n_els,
+                                uint32_t first, const ScatPackPlan& plan, int row_bytes, void* out, uint64_t* starts,
+                                hipStream_t s) {
+  if (n == 0 || n_els == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_row_starts, dim3(1), dim3(1024), 0, s, els, n_els, starts);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  uint64_t blocks = (n + 255) / 256;
+  if (blocks > 4096) blocks = 4096;
+  hipLaunchKernelGGL(k_order_scatter, dim3((unsigned)blocks), dim3(256), 0, s, rows, n, n_els, first, plan, row_bytes,
+                     starts, reinterpret_cast<uint8_t*>(out));
+  return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // host-side launchers
 

@@ -433,7 +433,8 @@ static hipError_t window_ds(const DevCfg& c, const RunArgs& R, int lg, hipStream
   const size_t lds = window_lds_bytes(c);
   const uint64_t per = kWinBlock >> lg;
   const uint64_t grid = (R.n + per - 1) / per;
-  const void* k = reinterpret_cast<const void*>(&k_window_ds<NCH, false>);
+  const void* k = R.rows ? reinterpret_cast<const void*>(&k_window_ds<NCH, true>)
+                         : reinterpret_cast<const void*>(&k_window_ds<NCH, false>);
   void* args[] = {(void*)&c, (void*)&R, (void*)&lg};
   return hipLaunchKernel(k, dim3((unsigned)grid), dim3(kWinBlock), args, lds, s);
 }
