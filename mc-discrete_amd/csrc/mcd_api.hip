@@ -1102,10 +1102,10 @@ static int forward_impl(mcd_ctx* ctx, const mcd_config* cfg, const mcd_tables* t
   const uint64_t want = (n + block - 1) / block;
   // launches too small to fill the chip with one lane per electron take
   // several lanes per electron, unless a placement or a shape is asked for
-  const int wlg = ds32 && !guard_flags && !shape_given ? window_log2_lanes(c, n, ctx->n_cu) : 0;
+  const int wlg = !guard_flags && !shape_given ? window_log2_lanes(c, precision, n, ctx->n_cu) : 0;
   if (wlg) {
     HIP_TRY(ctx, launch_fill_u64(q, 0ull, 1, s));
-    HIP_TRY(ctx, launch_window_ds(c, R, wlg, s));
+    HIP_TRY(ctx, launch_window(c, R, precision, wlg, s));
   } else if (service) {
     // wavefront 0 of each workgroup serves the guard; the others carry electrons
     const uint64_t want_svc = (n + (uint64_t)(block - 64) - 1) / (uint64_t)(block - 64);

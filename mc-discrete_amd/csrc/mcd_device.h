@@ -286,21 +286,60 @@ __device__ __forceinline__ double d_sorted_probs(const double* sig, int n, int* 
 }
 
 // Exact FP64 pick: returns the channel label; also the FP64 mean free path.
-__device__ __noinline__ int d_pick(double E, double u, const DevCfg& c, double* mfp_out) {
-  double sig[MCD_MAX_CHANNELS], probs[MCD_MAX_CHANNELS];
-  int lab[MCD_MAX_CHANNELS], order[MCD_MAX_CHANNELS];
-  int n = d_sigma_set(E, c, sig, lab);
-  double s = 0.;
-  for (int i = 0; i < n; ++i) s += sig[i];
-  *mfp_out = 1. / (c.atnd * s) * 1e14;  // mfp_from_sigma, scattering.py:19-36
-  d_sorted_probs(sig, n, order, probs);
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    if (probs[mid] < u) lo = mid + 1; else hi = mid;
+// The sigma set, its stable descending sort (a network of adjacent exchanges)
+// and the cumulative sums stay in registers (indexed arrays are scratch
+// memory: a step took 18 us on a lone wavefront, 2.4 us now).  probs[k] < u,
+// the cumulative sum over the total, is decided from cum - u total where that
+// is not near zero and by the division otherwise.
+template <int NCH>
+__device__ __forceinline__ int d_pick(double E, double u, const DevCfg& c, double* mfp_out) {
+  double sig[NCH];
+  int idx[NCH];
+  sig[0] = d_sigma_ruth(E, c);
+  sig[1] = d_sigma_moller(E, c);
+#pragma unroll
+  for (int s = 0; s < NCH - 3; ++s) sig[2 + s] = d_sigma_gryz(E, c.Eb[s], c.ns[s]);
+  sig[NCH - 1] = d_sigma_quinn(E, c);
+  double sum = 0.;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    sum += sig[i];
+    idx[i] = i;
   }
-  if (lo >= n) lo = n - 1;
-  return lab[order[lo]];
+  *mfp_out = 1. / (c.atnd * sum) * 1e14;  // mfp_from_sigma, scattering.py:19-36
+#pragma unroll
+  for (int i = 1; i < NCH; ++i) {
+#pragma unroll
+    for (int j = i; j > 0; --j) {
+      const bool sw = sig[j - 1] < sig[j];
+      const double a = sig[j - 1], b = sig[j];
+      const int ia = idx[j - 1], ib = idx[j];
+      sig[j - 1] = sw ? b : a;
+      sig[j] = sw ? a : b;
+      idx[j - 1] = sw ? ib : ia;
+      idx[j] = sw ? ia : ib;
+    }
+  }
+#pragma unroll
+  for (int i = 1; i < NCH; ++i) sig[i] += sig[i - 1];
+  const double tot = sig[NCH - 1], ut = u * tot, near_ = 1e-15 * tot;
+  uint32_t below = 0;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const double d = sig[i] - ut;
+    bool lt = d < 0.;
+    if (!(tot > 0. && fabs(d) > near_)) lt = sig[i] / tot < u;
+    below |= lt ? 1u << i : 0u;
+  }
+  int lo = 0, hi = NCH;  // bisect_left
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if ((below >> mid) & 1u) lo = mid + 1; else hi = mid;
+  }
+  int i = idx[0];
+#pragma unroll
+  for (int q = 1; q < NCH; ++q) i = (lo == q || (q == NCH - 1 && lo > q)) ? idx[q] : i;
+  return i == 0 ? MCD_CH_RUTH : (i == 1 ? MCD_CH_MOLLER : (i == NCH - 1 ? MCD_CH_QUINN : MCD_CH_GRYZ0 + i - 2));
 }
 #pragma clang fp contract(off)
 // Sigma of one channel label in FP64 (one formula per call keeps the guard
@@ -592,9 +631,17 @@ __device__ __forceinline__ void f_rotate(float c2, float s2, float u_az, float* 
 #pragma clang fp contract(off)
 // FP64 rotation as the reference composes it: Hamilton product, rotation
 // matrix normalised by |q|^2, renormalisation of both vectors.
-__device__ __forceinline__ void d_rotate(double c2, double halfPhi, double* d, double* y) {
-  double s_ht = pow(1. - c2, 0.5), c_ht = pow(c2, 0.5);
-  double s_hp = sin(halfPhi), c_hp = pow(1. - s_hp * s_hp, 0.5);
+// Cosine and sine of the half angles first (of the polar angle from its
+// cos^2, of the folded azimuth from halfPhi).
+__device__ __forceinline__ void d_half_angles(double c2, double halfPhi, double& c_ht, double& s_ht, double& c_hp,
+                                              double& s_hp) {
+  s_ht = sqrt(1. - c2);
+  c_ht = sqrt(c2);
+  s_hp = sin(halfPhi);
+  c_hp = sqrt(1. - s_hp * s_hp);
+}
+
+__device__ __forceinline__ void d_rotate(double c_ht, double s_ht, double c_hp, double s_hp, double* d, double* y) {
   double a1 = c_hp, b1 = d[0] * s_hp, c1 = d[1] * s_hp, d1 = d[2] * s_hp;
   double a2 = c_ht, b2 = y[0] * s_ht, c2q = y[1] * s_ht, d2 = y[2] * s_ht;
   double w = a1 * a2 - b1 * b2 - c1 * c2q - d1 * d2;

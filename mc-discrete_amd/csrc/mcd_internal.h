@@ -99,9 +99,9 @@ int max_blocks_per_cu(const DevCfg& c, int precision, int minw, int block);
 // DS FP32 with the FP64 guard deferred: phase 1 parks guarded steps, phase 2 resumes them
 hipError_t launch_transport_deferred(const DevCfg& c, const RunArgs& R, int phase, int grid, int block, hipStream_t s);
 int deferred_blocks_per_cu(const DevCfg& c, int phase, int block);
-// DS FP32, small launches: 2^lg lanes per electron (mcd_window.hip)
-int window_log2_lanes(const DevCfg& c, uint64_t n, int n_cu);
-hipError_t launch_window_ds(const DevCfg& c, const RunArgs& R, int lg, hipStream_t s);
+// small launches: 2^lg lanes per electron (mcd_window.hip)
+int window_log2_lanes(const DevCfg& c, int precision, uint64_t n, int n_cu);
+hipError_t launch_window(const DevCfg& c, const RunArgs& R, int precision, int lg, hipStream_t s);
 // DS FP32 with the FP64 guard served by wavefront 0 of each workgroup
 hipError_t launch_transport_svc(const DevCfg& c, const RunArgs& R, int minw, int grid, int block, hipStream_t s);
 int svc_blocks_per_cu(const DevCfg& c, int minw, int block);

@@ -156,4 +156,114 @@ __device__ __forceinline__ void ds_loss_angles(const DevCfg& c, const DevTable* 
   }
 }
 
+// Free path l, loss Wh + Wl and Joy's screening parameter a (the polar angle's)
+// of a continuous-mode step; ln_u0 = ln of the path's random number.  EXPL:
+// the explicit Bethe law, evaluated in FP64.
+template <bool EXPL>
+__device__ __forceinline__ void cont_path_loss(const DevCfg& c, F2 E, float ln_u0, float& a, float& l, float& Wh,
+                                               float& Wl, uint32_t& sflags) {
+  Wl = 0.f;
+  // Rutherford-only mean free path (scattering.py:780-797)
+  // Joy's screening: the polar angle (Rutherford_halfPol) in every model
+  a = c.c_alpha_f * __builtin_amdgcn_rcpf(E.hi);
+  float sig;
+  if (c.elastic >= MCD_ELASTIC_NIGRAM) {  // ruther_N_sigma(_wDefl), crossSections.py:91-147
+    const float b = 0.48f * (c.nig_zp_f * __builtin_amdgcn_rcpf(E.hi));
+    sig = c.nig_num_f * __builtin_amdgcn_rcpf(4.f * b * (1.f + b) * (E.hi * E.hi));
+  } else {
+    const float Ek = E.hi * 1e-3f;
+    const float rr = (Ek + 511.f) * __builtin_amdgcn_rcpf(Ek + 1024.f);
+    sig = c.ruth_k_f * rr * rr * __builtin_amdgcn_rcpf(Ek * Ek * a * (1.f + a));
+  }
+  const float mfp = c.mfp_k_f * __builtin_amdgcn_rcpf(sig);
+  l = -mfp * ln_u0;
+  if (!(l < 1e4f)) sflags |= MCD_FLAG_LONG_PATH;
+  // Bethe stopping power at the pre-step energy (stoppingPowers.py:112-215)
+  if constexpr (EXPL) {
+    // explicit law (:177-215), its shell sum folded to Z_eff (ln E - ln E*),
+    // in FP64: near Emin ln E and ln E* are close, and their FP32
+    // difference would lose most of its bits; the loss l*S is kept as a pair
+    const double Ed = (double)E.hi + (double)E.lo;
+    const double Wd = (double)l * (c.expl_k * (log(Ed) - c.lnEstar) / Ed);
+    Wh = (float)Wd;
+    Wl = (float)(Wd - (double)Wh);
+  } else {
+    float S;
+    const float iE = __builtin_amdgcn_rcpf(E.hi);
+    if (c.bethe == MCD_BETHE_CLASSICAL) S = c.bethe_k1_f * iE * ln_f(c.bethe_c1_f * E.hi);
+    else S = c.bethe_k1_f * iE * ln_f(c.bethe_c1_f * (E.hi + c.bethe_kJ_f));
+    Wh = l * S;
+  }
+  if (!f_lt_f2(Wh, E)) sflags |= MCD_FLAG_LOSS_GE_E;
+}
+
+// FP64 step: every quantity in double and the exact pick.  Arithmetic is not
+// contracted into FMAs so the operation order matches the reference expressions.
+struct DStep {
+  double l, W, c2, hp;
+  int ch;
+  uint32_t sflags;
+};
+
+#pragma clang fp contract(off)
+// One step's physics in FP64; tm, tg: the two loss tables (NCH channels, DS).
+template <int MODE, int NCH>
+__device__ __forceinline__ DStep d_step_physics(const DevCfg& c, const DevTable& tm, const DevTable& tg, double E,
+                                                const U4 r) {
+  DStep o;
+  o.sflags = 0;
+  o.ch = MCD_CH_RUTH;
+  if (MODE == MCD_MODE_DS) {
+    const double u0 = u01d(r.x), u1 = u01d(r.y), u2 = u01d(r.z), u3 = u01d(r.w);
+    double mfp;
+    o.ch = d_pick<NCH>(E, u0, c, &mfp);          // det_type, scattering.py:530-549
+    o.l = -mfp * log(u1);                   // compute_pathl, :551-565
+    if (o.ch == MCD_CH_RUTH) {              // :575-586
+      o.W = 0.;
+      const double a = c.c_alpha / E;
+      o.c2 = 1. - (a * u2 / (1. + a - u2));
+    } else if (o.ch == MCD_CH_QUINN) {      // :643-656
+      o.W = c.Epl;
+      o.c2 = 1.;
+    } else {                                // :602-640
+      const DevTable& t = (o.ch == MCD_CH_MOLLER) ? tm : tg;
+      const double Ec = E;
+      int row;
+      const int col = table_lookup(t, (float)E, [Ec](float v) { return (double)v < Ec; }, (float)u2, row);
+      o.W = (double)ldg(t.Ws + col);
+      if (!(o.W < E)) o.sflags |= MCD_FLAG_LOSS_GE_E;
+      if (o.W <= (E - c.Ef) * 0.5) o.c2 = 0.5 * (sqrt(1 - (o.W / E)) + 1);
+      else { o.c2 = __builtin_nan(""); o.sflags |= MCD_FLAG_NAN_DIR; }
+    }
+    o.hp = kPi * u3;
+  } else {
+    const double u0 = u01d(r.x), u1 = u01d(r.y), u2 = u01d(r.z);
+    const double sr = d_sigma_ruth(E, c);
+    const double mfp = 1. / (c.atnd * sr) * 1e14;  // scattering.py:792
+    o.l = -mfp * log(u0);                          // :802-813
+    if (!(o.l < 1e4)) o.sflags |= MCD_FLAG_LONG_PATH;
+    double S;                                      // stoppingPowers.py:112-215
+    if (c.bethe == MCD_BETHE_CLASSICAL) S = 2. * kPiEFour * c.atnd * ((double)c.Z / E) * log(1.166 * (E) / c.J) * 1e-14;
+    else if (c.bethe == MCD_BETHE_JL)
+      S = 2. * kPiEFour * c.atnd * ((double)c.Z / E) * log(1.166 * (E + c.bethe_kk * c.J) / c.J) * 1e-14;
+    else {
+      const double pref = (2. * kPiEFour * c.atnd / E) * 1e-14;
+      double sumi = c.n_val * log(E * 1. / c.E_val);
+      for (int i = 0; i < c.n_shells; ++i) sumi = sumi + c.ns[i] * log(E * 1. / c.Eb[i]);
+      S = pref * sumi;
+    }
+    o.W = o.l * S;                                 // compute_Eloss, :815-826
+    if (!(o.W < E)) o.sflags |= MCD_FLAG_LOSS_GE_E;
+    const double a = c.c_alpha / E;                // compute_sAngles, :828-840
+    o.c2 = 1. - (a * u1 / (1. + a - u1));
+    o.hp = kPi * u2;
+  }
+  return o;
+}
+
+__device__ __forceinline__ void d_advance(const double* p, double l, const double* d, double* np_) {
+  for (int i = 0; i < 3; ++i) np_[i] = p[i] + l * d[i];
+}
+#pragma clang fp contract(on)
+
 }  // namespace mcd

@@ -295,38 +295,8 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
     } else {
       const float u0 = u01f(r.x), u1 = u01f(r.y);
       u_az = u01f(r.z);
-      // Rutherford-only mean free path (scattering.py:780-797)
-      // Joy's screening: the polar angle (Rutherford_halfPol) in every model
-      const float a = c.c_alpha_f * __builtin_amdgcn_rcpf(E.hi);
-      float sig;
-      if (c.elastic >= MCD_ELASTIC_NIGRAM) {  // ruther_N_sigma(_wDefl), crossSections.py:91-147
-        const float b = 0.48f * (c.nig_zp_f * __builtin_amdgcn_rcpf(E.hi));
-        sig = c.nig_num_f * __builtin_amdgcn_rcpf(4.f * b * (1.f + b) * (E.hi * E.hi));
-      } else {
-        const float Ek = E.hi * 1e-3f;
-        const float rr = (Ek + 511.f) * __builtin_amdgcn_rcpf(Ek + 1024.f);
-        sig = c.ruth_k_f * rr * rr * __builtin_amdgcn_rcpf(Ek * Ek * a * (1.f + a));
-      }
-      const float mfp = c.mfp_k_f * __builtin_amdgcn_rcpf(sig);
-      l = -mfp * ln_f(u0);
-      if (!(l < 1e4f)) sflags |= MCD_FLAG_LONG_PATH;
-      // Bethe stopping power at the pre-step energy (stoppingPowers.py:112-215)
-      if constexpr (EXPL) {
-        // explicit law (:177-215), its shell sum folded to Z_eff (ln E - ln E*),
-        // in FP64: near Emin ln E and ln E* are close, and their FP32
-        // difference would lose most of its bits; the loss l*S is kept as a pair
-        const double Ed = (double)E.hi + (double)E.lo;
-        const double Wd = (double)l * (c.expl_k * (log(Ed) - c.lnEstar) / Ed);
-        Wh = (float)Wd;
-        Wl = (float)(Wd - (double)Wh);
-      } else {
-        float S;
-        const float iE = __builtin_amdgcn_rcpf(E.hi);
-        if (c.bethe == MCD_BETHE_CLASSICAL) S = c.bethe_k1_f * iE * ln_f(c.bethe_c1_f * E.hi);
-        else S = c.bethe_k1_f * iE * ln_f(c.bethe_c1_f * (E.hi + c.bethe_kJ_f));
-        Wh = l * S;
-      }
-      if (!f_lt_f2(Wh, E)) sflags |= MCD_FLAG_LOSS_GE_E;
+      float a;
+      cont_path_loss<EXPL>(c, E, ln_f(u0), a, l, Wh, Wl, sflags);
       const float om = 1.f - u1;
       const float inv = __builtin_amdgcn_rcpf(om + a);
       s2 = a * u1 * inv;
@@ -754,72 +724,8 @@ hipError_t launch_count_outcomes_batched(const BatchItemDev* items, int n_items,
 // FP64 transport: the same loop with every quantity in double and the exact
 // pick each step (the all-FP64 GPU run).  Arithmetic is not contracted into
 // FMAs so the operation order matches the reference expressions.
-struct DStep {
-  double l, W, c2, hp;
-  int ch;
-  uint32_t sflags;
-};
 
-#pragma clang fp contract(off)
-template <int MODE>
-__device__ __forceinline__ DStep d_step_physics(const DevCfg& c, double E, const U4 r) {
-  DStep o;
-  o.sflags = 0;
-  o.ch = MCD_CH_RUTH;
-  if (MODE == MCD_MODE_DS) {
-    const double u0 = u01d(r.x), u1 = u01d(r.y), u2 = u01d(r.z), u3 = u01d(r.w);
-    double mfp;
-    o.ch = d_pick(E, u0, c, &mfp);          // det_type, scattering.py:530-549
-    o.l = -mfp * log(u1);                   // compute_pathl, :551-565
-    if (o.ch == MCD_CH_RUTH) {              // :575-586
-      o.W = 0.;
-      const double a = c.c_alpha / E;
-      o.c2 = 1. - (a * u2 / (1. + a - u2));
-    } else if (o.ch == MCD_CH_QUINN) {      // :643-656
-      o.W = c.Epl;
-      o.c2 = 1.;
-    } else {                                // :602-640
-      const DevTable& t = (o.ch == MCD_CH_MOLLER) ? c.tm : c.tg;
-      const double Ec = E;
-      int row;
-      const int col = table_lookup(t, (float)E, [Ec](float v) { return (double)v < Ec; }, (float)u2, row);
-      o.W = (double)t.Ws[col];
-      if (!(o.W < E)) o.sflags |= MCD_FLAG_LOSS_GE_E;
-      if (o.W <= (E - c.Ef) * 0.5) o.c2 = 0.5 * (sqrt(1 - (o.W / E)) + 1);
-      else { o.c2 = __builtin_nan(""); o.sflags |= MCD_FLAG_NAN_DIR; }
-    }
-    o.hp = kPi * u3;
-  } else {
-    const double u0 = u01d(r.x), u1 = u01d(r.y), u2 = u01d(r.z);
-    const double sr = d_sigma_ruth(E, c);
-    const double mfp = 1. / (c.atnd * sr) * 1e14;  // scattering.py:792
-    o.l = -mfp * log(u0);                          // :802-813
-    if (!(o.l < 1e4)) o.sflags |= MCD_FLAG_LONG_PATH;
-    double S;                                      // stoppingPowers.py:112-215
-    if (c.bethe == MCD_BETHE_CLASSICAL) S = 2. * kPiEFour * c.atnd * ((double)c.Z / E) * log(1.166 * (E) / c.J) * 1e-14;
-    else if (c.bethe == MCD_BETHE_JL)
-      S = 2. * kPiEFour * c.atnd * ((double)c.Z / E) * log(1.166 * (E + c.bethe_kk * c.J) / c.J) * 1e-14;
-    else {
-      const double pref = (2. * kPiEFour * c.atnd / E) * 1e-14;
-      double sumi = c.n_val * log(E * 1. / c.E_val);
-      for (int i = 0; i < c.n_shells; ++i) sumi = sumi + c.ns[i] * log(E * 1. / c.Eb[i]);
-      S = pref * sumi;
-    }
-    o.W = o.l * S;                                 // compute_Eloss, :815-826
-    if (!(o.W < E)) o.sflags |= MCD_FLAG_LOSS_GE_E;
-    const double a = c.c_alpha / E;                // compute_sAngles, :828-840
-    o.c2 = 1. - (a * u1 / (1. + a - u1));
-    o.hp = kPi * u2;
-  }
-  return o;
-}
-
-__device__ __forceinline__ void d_advance(const double* p, double l, const double* d, double* np_) {
-  for (int i = 0; i < 3; ++i) np_[i] = p[i] + l * d[i];
-}
-#pragma clang fp contract(on)
-
-template <int MODE>
+template <int MODE, int NCH>
 __global__ __launch_bounds__(256) void k_transport_f64(DevCfg c, RunArgs R) {
   const int lane = threadIdx.x & 63;
   const uint32_t k0 = (uint32_t)R.seed, k1 = (uint32_t)(R.seed >> 32);
@@ -858,7 +764,7 @@ __global__ __launch_bounds__(256) void k_transport_f64(DevCfg c, RunArgs R) {
     }
     const U4 r = philox10((uint32_t)e, c.config_id | (uint32_t)(e >> 32) << 16, step, 0u, k0, k1);
     const double Epre = E;
-    const DStep o = d_step_physics<MODE>(c, E, r);
+    const DStep o = d_step_physics<MODE, NCH>(c, c.tm, c.tg, E, r);
     n_events++;
     double np_[3];
     d_advance(p, o.l, d, np_);
@@ -880,7 +786,11 @@ __global__ __launch_bounds__(256) void k_transport_f64(DevCfg c, RunArgs R) {
       write_rec(&R.els[e - R.first], (float)Epre, df, pf, step + 1, o1, o2, flags);
     }
     const bool rec_row = R.rows != nullptr && e < R.row_max_electron;
-    if (!done || rec_row) d_rotate(o.c2, o.hp, d, y);
+    if (!done || rec_row) {
+      double c_ht, s_ht, c_hp, s_hp;
+      d_half_angles(o.c2, o.hp, c_ht, s_ht, c_hp, s_hp);
+      d_rotate(c_ht, s_ht, c_hp, s_hp, d, y);
+    }
     if (R.rows != nullptr) {
       const uint64_t slot = append_slot(rec_row, R.row_cursor, R.row_cap, lane);
       if (slot != ~0ull) {
@@ -1068,14 +978,26 @@ static hipError_t dispatch_f32(int minw, const DevCfg& c, const RunArgs* R, int 
 
 bool valid_minw(int w) { return w == 1 || w == 4 || w == 5 || w == 6 || w == 8; }
 
+// the FP64 kernel of a configuration
+static const void* f64_kernel(const DevCfg& c) {
+  if (c.mode != MCD_MODE_DS) return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_CONT, 4>);
+  switch (c.n_shells + 3) {
+    case 4: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 4>);
+    case 5: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 5>);
+    case 6: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 6>);
+    case 7: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 7>);
+    case 8: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 8>);
+    case 9: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 9>);
+    case 10: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 10>);
+    default: return reinterpret_cast<const void*>(&k_transport_f64<MCD_MODE_DS, 11>);
+  }
+}
+
 hipError_t launch_transport(const DevCfg& c, const RunArgs& R, int precision, int minw, int grid, int block,
                             hipStream_t s) {
   if (precision == MCD_PREC_FP64) {
-    if (c.mode == MCD_MODE_DS)
-      hipLaunchKernelGGL((k_transport_f64<MCD_MODE_DS>), dim3(grid), dim3(block), 0, s, c, R);
-    else
-      hipLaunchKernelGGL((k_transport_f64<MCD_MODE_CONT>), dim3(grid), dim3(block), 0, s, c, R);
-    return hipGetLastError();
+    void* args[] = {(void*)&c, (void*)&R};
+    return hipLaunchKernel(f64_kernel(c), dim3(grid), dim3(block), args, 0, s);
   }
   return dispatch_f32(minw, c, &R, grid, block, s, nullptr);
 }
@@ -1084,10 +1006,7 @@ hipError_t launch_transport(const DevCfg& c, const RunArgs& R, int precision, in
 int max_blocks_per_cu(const DevCfg& c, int precision, int minw, int block) {
   int nb = 1;
   if (precision == MCD_PREC_FP64) {
-    hipError_t e = c.mode == MCD_MODE_DS
-                       ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_transport_f64<MCD_MODE_DS>, block, 0)
-                       : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_transport_f64<MCD_MODE_CONT>, block, 0);
-    if (e != hipSuccess || nb < 1) nb = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f64_kernel(c), block, 0) != hipSuccess || nb < 1) nb = 1;
     return nb;
   }
   if (dispatch_f32(minw, c, nullptr, 0, block, 0, &nb) != hipSuccess || nb < 1) nb = 1;

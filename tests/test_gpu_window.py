@@ -17,6 +17,11 @@ def _transport(material="Cu", E0=20000.0, Emin=1000.0, Wc=50.0, tilt=70.0, **kw)
     return engine.Transport(material, E0, Emin, Wc=Wc, s_tilt=tilt, tol_E=1e-2, tol_W=1e-2, grid_search="library", **kw)
 
 
+# FP64 kernels and continuous mode have one form for an explicit block
+ONE_LANE = dict(block=256)
+FP64 = _abi.PREC_FP64
+
+
 def _same(a, b):
     assert a.els.tobytes() == b.els.tobytes()
     assert np.array_equal(a.counters[COUNTED], b.counters[COUNTED])
@@ -62,3 +67,44 @@ def test_repeated_runs_are_equal(cu):
     a = cu.run(12345, seed=8)
     for _ in range(3):
         _same(cu.run(12345, seed=8), a)
+
+
+# FP64 (DS): 1.5 wavefronts per SIMD to 8 lanes (98304 lanes), 4 to 4 lanes
+@pytest.mark.parametrize("n", [1, 65, 1536, 1537, 12289, 65537])
+def test_fp64_sizes_equal_one_lane_per_electron(cu, n):
+    _same(cu.run(n, seed=n, precision=FP64), cu.run(n, seed=n, precision=FP64, **ONE_LANE))
+
+
+@pytest.mark.parametrize("kw", [
+    dict(material="Al", E0=5000.0, Emin=500.0, tilt=0.0, thickness=2000.0),
+    dict(material="Au", E0=5000.0, Wc=20.0, elastic="Ruth_nigram"),
+    dict(max_scatt=64), dict(max_scatt=1),
+], ids=str)
+def test_fp64_configurations_and_rows_equal_one_lane_per_electron(kw):
+    tr = _transport(**kw)
+    kw = dict(seed=3, first=(1 << 32) - 7, precision=FP64)
+    _same(tr.run(1200, **kw), tr.run(1200, **kw, **ONE_LANE))
+    kw.update(scats=True)
+    _same(tr.run(40, **kw), tr.run(40, **kw, **ONE_LANE))
+
+
+# continuous mode: one wavefront per SIMD (65536 lanes), quads to two (explicit law: to one)
+@pytest.mark.parametrize("law", ["classical", "JL", "explicit"])
+@pytest.mark.parametrize("n", [1, 65, 1024, 1025, 8193, 16384, 16385, 32769])
+def test_continuous_sizes_equal_one_lane_per_electron(law, n):
+    tr = engine.Transport("Au", 10000.0, 1000.0, s_tilt=70.0, mode="cont", bethe_model=law)
+    _same(tr.run(n, seed=n), tr.run(n, seed=n, **ONE_LANE))
+
+
+@pytest.mark.parametrize("kw", [
+    dict(material="Cu", bethe_model="classical", thickness=20000.0, s_tilt=0.0),
+    dict(material="Al", bethe_model="JL", elastic="Ruth_nigram", max_scatt=17),
+    dict(material="Au", bethe_model="explicit", max_scatt=1),
+    dict(material="Si", bethe_model="JL", thickness=800.0, max_scatt=64),
+], ids=str)
+def test_continuous_configurations_and_rows_equal_one_lane_per_electron(kw):
+    tr = engine.Transport(kw.pop("material"), 10000.0, 1000.0, mode="cont", **{"s_tilt": 60.0, **kw})
+    for n in (33, 9000):
+        _same(tr.run(n, seed=3, first=9), tr.run(n, seed=3, first=9, **ONE_LANE))
+    _same(tr.run(70, seed=3, scats=True, scat_max_electron=50), tr.run(70, seed=3, scats=True, scat_max_electron=50,
+                                                                      **ONE_LANE))
