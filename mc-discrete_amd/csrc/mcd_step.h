@@ -10,6 +10,29 @@
 
 namespace mcd {
 
+// Kernel arguments read anew where a rare path uses them.  The compiler cannot
+// tell these loads from others, so it neither hoists what the path computes
+// from them out of a loop nor keeps their values for it: in the inline-guard
+// kernel the FP64 pick's constants took 40 SGPRs and VGPRs of every step.
+template <class T>
+using Const4 = const __attribute__((address_space(4))) T;
+// The arguments of a kernel that takes (DevCfg, RunArgs, ..).
+struct KernelArgs {
+  DevCfg c;
+  RunArgs R;
+};
+__device__ __forceinline__ const KernelArgs& args_anew() {
+  Const4<KernelArgs>* p = (Const4<KernelArgs>*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return (const KernelArgs&)*p;
+}
+// A configuration in the constant address space (a batch item's).
+__device__ __forceinline__ const DevCfg& cfg_anew(const DevCfg& c) {
+  Const4<DevCfg>* p = (Const4<DevCfg>*)&c;
+  asm volatile("" : "+s"(p));
+  return (const DevCfg&)*p;
+}
+
 // LDS of the one-configuration kernels: the pick table (nf floats), then the
 // two loss-table descriptors at a 16-byte aligned offset.
 __host__ __device__ constexpr int tab_offset_floats(int nf) { return (nf + 3) & ~3; }

@@ -9,9 +9,12 @@
 // numerics.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mcd_device.h"
 #include "mcd_internal.h"
 #include "mcd_step.h"
+#include "mcd_window.h"
 
 namespace mcd {
 
@@ -137,11 +140,15 @@ __device__ void guard_service(const DevCfg& c, GuardBox* boxes, uint32_t* pendin
 // Philox counter.  PHASE 3 (DS): guard-band picks go to the workgroup's
 // service wavefront through `box`; same records as phase 0.
 // EXPL (continuous mode): the explicit Bethe law, evaluated in FP64.
-template <int MODE, int NCH, int PHASE = 0, bool PERIOD = false, bool EXPL = false, bool WIDE = false>
+// ITEM: c is a batch item's configuration, not the kernel's argument.
+// DRAIN: once the work counter is spent and at most R.drain lanes are left, the
+// loop ends and hands them over in `rest`.
+template <int MODE, int NCH, int PHASE = 0, bool PERIOD = false, bool EXPL = false, bool WIDE = false,
+          bool DRAIN = false, bool ITEM = false>
 __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __restrict__ lds,
                                                const DevTable* __restrict__ tabs, const RunArgs& R,
                                                uint32_t& n_events, uint32_t& n_fp64, GuardBox* box = nullptr,
-                                               uint32_t* pending = nullptr) {
+                                               uint32_t* pending = nullptr, LaneEl* rest = nullptr) {
   const int lane = threadIdx.x & 63;
   uint32_t k0 = (uint32_t)R.seed, k1 = (uint32_t)(R.seed >> 32);
   const uint64_t n_work = PHASE == 2 ? (uint64_t)__atomic_load_n(R.park_count, __ATOMIC_RELAXED) : R.n;
@@ -199,6 +206,23 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
             }
           }
         }
+      }
+    }
+    if constexpr (DRAIN) {
+      if (!open && __popcll(__ballot(active)) <= R.drain) {
+        rest->active = active;
+        rest->e = e;
+        rest->step = step;
+        rest->flags = flags;
+        rest->E = E;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          rest->p[i] = p[i];
+          rest->pc[i] = pc[i];
+          rest->d[i] = d[i];
+          rest->y[i] = y[i];
+        }
+        break;
       }
     }
     if (!__any(active)) break;
@@ -285,7 +309,8 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
         if (ch < 0) {  // guard band: settle the pick in FP64
           uint32_t plo, phi;
           guard_perm<NCH>(pe, plo, phi);
-          ch = d_pick_ordered<NCH>((double)E.hi + (double)E.lo, (double)u0, c, plo, phi, pe.swap, pe.exact);
+          const DevCfg& ca = ITEM ? cfg_anew(c) : args_anew().c;
+          ch = d_pick_ordered<NCH>((double)E.hi + (double)E.lo, (double)u0, ca, plo, phi, pe.swap, pe.exact);
           sflags |= MCD_FLAG_FP64_PICK;
           n_fp64++;
         }
@@ -358,7 +383,19 @@ __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R
     __syncthreads();
   }
   uint32_t n_events = 0, n_fp64 = 0;
-  transport_loop<MODE, NCH, PHASE, true, EXPL>(c, lds, tabs, R, n_events, n_fp64);
+  constexpr bool drain = PHASE == 0 && MINW == 4;
+  LaneEl rest;
+  transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain>(c, lds, tabs, R, n_events, n_fp64, nullptr, nullptr,
+                                                             &rest);
+  if constexpr (drain) {
+    typedef typename std::conditional<MODE == MCD_MODE_DS, Fp32Ds<NCH>, Fp32Cont<EXPL>>::type P;
+    // The arguments read anew: shared with the loop above, the drain's uses
+    // made the loop reload or spill its scalars at every step (5 % slower).
+    const KernelArgs& A = args_anew();
+    typename P::Staged* win = reinterpret_cast<typename P::Staged*>(reinterpret_cast<char*>(lds) + A.R.win_off) +
+                              win_stage(1) * (threadIdx.x >> 6);
+    if (A.R.drain) window_drain<P>(A.c, A.R, lds, tabs, win, rest, n_events, n_fp64);
+  }
   const int lane = threadIdx.x & 63;
   const uint64_t cnt[2] = {n_events, n_fp64};
   wave_add_counters(R.counters + MCD_CNT_EVENTS, cnt, 1, lane);
@@ -491,7 +528,8 @@ __device__ __forceinline__ void run_item(const DevCfg& c, const DevCfg& cl, cons
   // the item's counter block of this launch: phases 2 and 3 count errors in it
   if constexpr (PHASE >= 2) R.counters = ic;
   // the table descriptors from the LDS copy: the per-lane Moller / Gryzinski select reads LDS
-  transport_loop<MODE, NCH, MODE == MCD_MODE_DS ? PHASE : 0, PERIOD, EXPL>(c, pick, &cl.tm, R, ne, nf, box, pending);
+  transport_loop<MODE, NCH, MODE == MCD_MODE_DS ? PHASE : 0, PERIOD, EXPL, false, false, true>(
+      c, pick, &cl.tm, R, ne, nf, box, pending);
 }
 
 // The batched kernel's service wavefront: as guard_service, for mailboxes
@@ -926,15 +964,39 @@ hipError_t launch_order_scatter(const mcd_scatter_rec* rows, uint64_t n, const m
 // ---------------------------------------------------------------------------
 // host-side launchers
 
+// Electrons a wavefront goes on with in the window form once the work counter is
+// spent (one group of 4 lanes each).  Their last 1000 to 5000 steps cost 1.4 to
+// 1.9 us each with one lane per electron.  Launches of 2^20 electrons in us
+// without it and at 8 and 16: @@
+constexpr int kDrain = 16;
+
+// LDS of a one-kernel launch that needs `used` bytes for its step, with the
+// windows of its last electrons after them (D.win_off, D.drain); without them
+// where they would take the place of resident wavefronts (16 per CU at 4 per
+// SIMD, 160 KB of LDS).
+static size_t with_drain(size_t used, int block, RunArgs& D) {
+  const size_t at = (used + 15) & ~(size_t)15;
+  const size_t all = at + (size_t)(block / 64) * win_stage(1) * sizeof(Fp32Base::Staged);
+  const bool fits = all <= 64 * 1024 && all * (1024 / block) <= 160 * 1024;
+  D.win_off = (int)at;
+  D.drain = fits ? kDrain : 0;
+  return fits ? all : used;
+}
+
 template <int MODE, int NCH, int MINW, bool EXPL>
-static hipError_t launch_f32(const DevCfg& c, const RunArgs& R, int grid, int block, size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL((k_transport_f32<MODE, NCH, MINW, 0, EXPL>), dim3(grid), dim3(block), lds, s, c, R);
+static hipError_t launch_f32(const DevCfg& c, const RunArgs& R, int grid, int block, size_t used, hipStream_t s) {
+  RunArgs D = R;
+  const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
+  if (R.rows || MINW != 4) D.drain = 0;
+  hipLaunchKernelGGL((k_transport_f32<MODE, NCH, MINW, 0, EXPL>), dim3(grid), dim3(block), lds, s, c, D);
   return hipGetLastError();
 }
 
 template <int MODE, int NCH, int MINW, bool EXPL>
-static int occ_f32(int block, size_t lds) {
+static int occ_f32(int block, size_t used) {
   int nb = 0;
+  RunArgs D;
+  const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_transport_f32<MODE, NCH, MINW, 0, EXPL>, block, lds) !=
       hipSuccess)
     return 1;

@@ -108,3 +108,37 @@ def test_continuous_configurations_and_rows_equal_one_lane_per_electron(kw):
         _same(tr.run(n, seed=3, first=9), tr.run(n, seed=3, first=9, **ONE_LANE))
     _same(tr.run(70, seed=3, scats=True, scat_max_electron=50), tr.run(70, seed=3, scats=True, scat_max_electron=50,
                                                                       **ONE_LANE))
+
+
+# The last electrons of a large launch go on with several lanes each.  Forms
+# without that: wavefront budgets other than 4 per SIMD, the served guard.
+@pytest.mark.parametrize("kw", [
+    dict(),
+    dict(material="Au", E0=30000.0, Wc=20.0),
+    dict(material="Al", E0=5000.0, Emin=500.0, tilt=0.0, thickness=2000.0),
+    dict(max_scatt=65), dict(max_scatt=1),
+], ids=str)
+@pytest.mark.parametrize("n,first", [(81921, 0), (131073, (1 << 32) - 60000), (400000, 9)])
+def test_ds_drain_equals_one_lane_per_electron(kw, n, first):
+    tr = _transport(**kw)
+    a = tr.run(n, seed=4, first=first)
+    _same(a, tr.run(n, seed=4, first=first, waves_per_simd=5))
+    _same(tr.run(n, seed=4, first=first, block=64), a)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 700, 70000])
+def test_drain_of_small_inline_launches(cu, n):
+    _same(cu.run(n, seed=n, guard="inline"), cu.run(n, seed=n, guard="service"))
+    tr = _transport(material="Si", E0=10000.0, thickness=9000.0, tilt=0.0)
+    _same(tr.run(n, seed=n, guard="inline"), tr.run(n, seed=n, waves_per_simd=8))
+
+
+@pytest.mark.parametrize("kw", [
+    dict(material="Au", bethe_model="JL"), dict(material="Cu", bethe_model="classical", thickness=20000.0, s_tilt=0.0),
+    dict(material="Au", bethe_model="explicit"), dict(material="Al", bethe_model="JL", max_scatt=17),
+], ids=str)
+@pytest.mark.parametrize("n", [17, 32769, 200000])
+def test_continuous_drain_equals_one_lane_per_electron(kw, n):
+    kw = dict(kw)
+    tr = engine.Transport(kw.pop("material"), 10000.0, 1000.0, mode="cont", **{"s_tilt": 60.0, **kw})
+    _same(tr.run(n, seed=3, first=9, block=256), tr.run(n, seed=3, first=9, waves_per_simd=5))
