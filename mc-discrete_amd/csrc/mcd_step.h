@@ -289,4 +289,63 @@ __device__ __forceinline__ void d_advance(const double* p, double l, const doubl
 }
 #pragma clang fp contract(on)
 
+// ---------------------------------------------------------------------------
+// Service guard (DS, FP32, one kernel).  Wavefront 0 of a workgroup is a
+// service wavefront: a transport wavefront posts the guard-band picks of a step
+// to its LDS mailbox and waits; the service wavefront settles them in FP64, one
+// of its lanes per posted lane, and posts the channels back.  The FP64 code is
+// on a path no transport wavefront executes, so the kernel keeps the register
+// budget of an FP64-free step without a second kernel or a park buffer.
+struct GuardSlot {
+  float Ehi, Elo, u;
+  uint32_t perm_lo, perm_hi;
+  int meta;  // posted: swap position | exact << 8; replied: the channel
+};
+struct GuardBox {
+  unsigned long long mask;  // posted lanes
+  uint32_t state;           // kBoxPosted, then kBoxReplied
+  uint32_t bit;             // this mailbox's bit in the workgroup's pending word
+  GuardSlot lane[64];
+};
+constexpr uint32_t kBoxPosted = 1u, kBoxReplied = 2u;
+// A transport wavefront waits at most R.guard_spins s_sleep(2) polls for a
+// reply (kGuardSpinCap by default); past it the step takes the Rutherford
+// channel and is flagged MCD_FLAG_GUARD_TIMEOUT (counted as an error).
+
+__device__ __forceinline__ uint32_t box_load(const uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void box_store(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Post the picks with ch < 0 and wait for the channels (called by the active
+// lanes of a wavefront together).  sflags tells how a lane's pick was settled.
+template <int NCH>
+__device__ __forceinline__ void served_pick(GuardBox* box, uint32_t* pending, uint32_t max_spins, F2 E, float u0,
+                                            const PickEval<NCH>& pe, int& ch, uint32_t& sflags) {
+  const int lane = threadIdx.x & 63;
+  if (ch < 0) {
+    GuardSlot& g = box->lane[lane];
+    uint32_t plo, phi;
+    guard_perm<NCH>(pe, plo, phi);
+    g.Ehi = E.hi; g.Elo = E.lo; g.u = u0;
+    g.perm_lo = plo; g.perm_hi = phi;
+    g.meta = (pe.swap & 0xFF) | (pe.exact ? 0x100 : 0);
+  }
+  const uint64_t m = __ballot(ch < 0);
+  const int leader = __ffsll((unsigned long long)__ballot(true)) - 1;
+  if (lane == leader) {
+    box->mask = m;
+    box_store(&box->state, kBoxPosted);
+    __hip_atomic_fetch_or(pending, box->bit, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  uint32_t spins = 0;
+  while (box_load(&box->state) != kBoxReplied && ++spins < max_spins) __builtin_amdgcn_s_sleep(2);
+  if (ch < 0) {
+    ch = spins < max_spins ? box->lane[lane].meta : MCD_CH_RUTH;
+    sflags |= spins < max_spins ? MCD_FLAG_FP64_PICK : MCD_FLAG_GUARD_TIMEOUT;
+  }
+}
+
 }  // namespace mcd

@@ -55,35 +55,6 @@ __device__ __forceinline__ void count_outcome_words(const mcd_electron_rec* __re
 }
 
 // ---------------------------------------------------------------------------
-// Service guard (DS, FP32, one kernel).  Wavefront 0 of a workgroup is a
-// service wavefront: a transport wavefront posts the guard-band picks of a step
-// to its LDS mailbox and waits; the service wavefront settles them in FP64, one
-// of its lanes per posted lane, and posts the channels back.  The FP64 code is
-// on a path no transport wavefront executes, so the kernel keeps the register
-// budget of an FP64-free step without a second kernel or a park buffer.
-struct GuardSlot {
-  float Ehi, Elo, u;
-  uint32_t perm_lo, perm_hi;
-  int meta;  // posted: swap position | exact << 8; replied: the channel
-};
-struct GuardBox {
-  unsigned long long mask;  // posted lanes
-  uint32_t state;           // kBoxPosted, then kBoxReplied
-  uint32_t bit;             // this mailbox's bit in the workgroup's pending word
-  GuardSlot lane[64];
-};
-constexpr uint32_t kBoxPosted = 1u, kBoxReplied = 2u;
-// A transport wavefront waits at most R.guard_spins s_sleep(2) polls for a
-// reply (kGuardSpinCap by default); past it the step takes the Rutherford
-// channel and is flagged MCD_FLAG_GUARD_TIMEOUT (counted as an error).
-
-__device__ __forceinline__ uint32_t box_load(const uint32_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void box_store(uint32_t* p, uint32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 // The service wavefront's loop: answer posted mailboxes until every transport
 // wavefront of the workgroup has finished (each adds one to *done on exit;
 // a wavefront exits only after its last reply, so none is left waiting).
@@ -276,34 +247,9 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
         }
       } else if constexpr (PHASE == 3) {
         if (__any(ch < 0)) {  // guard band: post to the service wavefront and wait
-          if (ch < 0) {
-            GuardSlot& g = box->lane[lane];
-            uint32_t plo, phi;
-            guard_perm<NCH>(pe, plo, phi);
-            g.Ehi = E.hi; g.Elo = E.lo; g.u = u0;
-            g.perm_lo = plo; g.perm_hi = phi;
-            g.meta = (pe.swap & 0xFF) | (pe.exact ? 0x100 : 0);
-          }
-          const uint64_t m = __ballot(ch < 0);
-          const int leader = __ffsll((unsigned long long)__ballot(true)) - 1;
-          if (lane == leader) {
-            box->mask = m;
-            box_store(&box->state, kBoxPosted);
-            __hip_atomic_fetch_or(pending, box->bit, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-          }
-          uint32_t spins = 0;
-          while (box_load(&box->state) != kBoxReplied && ++spins < R.guard_spins) __builtin_amdgcn_s_sleep(2);
-          if (ch < 0) {
-            if (spins < R.guard_spins) {
-              ch = box->lane[lane].meta;
-              sflags |= MCD_FLAG_FP64_PICK;
-              n_fp64++;
-            } else {
-              ch = MCD_CH_RUTH;
-              sflags |= MCD_FLAG_GUARD_TIMEOUT;
-              atomicAdd(R.counters + MCD_CNT_GUARD_TIMEOUTS, 1ull);
-            }
-          }
+          served_pick<NCH>(box, pending, R.guard_spins, E, u0, pe, ch, sflags);
+          if (sflags & MCD_FLAG_FP64_PICK) n_fp64++;
+          if (sflags & MCD_FLAG_GUARD_TIMEOUT) atomicAdd(R.counters + MCD_CNT_GUARD_TIMEOUTS, 1ull);
         }
       } else {
         if (ch < 0) {  // guard band: settle the pick in FP64
@@ -402,25 +348,27 @@ __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R
   wave_add_counters(R.counters + MCD_CNT_FP64_PICKS, cnt + 1, 1, lane);
 }
 
-// Service-guard kernel (DS, FP32).  LDS: the pick table (wide records), the two loss-table
-// descriptors, one GuardBox per transport wavefront, the finished-wavefront
-// count and the pending-mailbox bits.  Wavefront 0 serves the guard picks, the others run the transport.
+// Service-guard kernel (DS, FP32).  LDS: one GuardBox per transport wavefront,
+// the finished-wavefront count and the pending-mailbox bits, the pick table
+// (wide records), the two loss-table descriptors.  Wavefront 0 serves the guard
+// picks, the others run the transport.
 // MINW: resident wavefronts per SIMD the register allocation must allow.
-__host__ __device__ inline size_t svc_box_offset(const DevCfg& c) {
-  return ((size_t)tab_offset_floats(c.pick.n_nodes * pick_stride_wide(c.pick.n_ch)) * sizeof(float) +
-          2 * sizeof(DevTable) + 15) &
-         ~(size_t)15;
+__host__ __device__ inline int svc_pick_offset(int block) {
+  return (int)(((block >> 6) - 1) * sizeof(GuardBox) + 16) / (int)sizeof(float);
 }
 static size_t svc_lds_bytes(const DevCfg& c, int block) {
-  return svc_box_offset(c) + (size_t)(block / 64 - 1) * sizeof(GuardBox) + 16;
+  return svc_pick_offset(block) * sizeof(float) +
+         (((size_t)tab_offset_floats(c.pick.n_nodes * pick_stride_wide(c.pick.n_ch)) * sizeof(float) +
+           2 * sizeof(DevTable) + 15) & ~(size_t)15);
 }
 
 template <int NCH, int MINW>
 __global__ __launch_bounds__(1024, MINW) void k_transport_svc(DevCfg c, RunArgs R) {
   extern __shared__ float lds[];
-  DevTable* tabs = stage_single_wide<NCH>(c, lds);
+  float* pick = lds + svc_pick_offset(blockDim.x);
+  DevTable* tabs = stage_single_wide<NCH>(c, pick);
   const int n_boxes = (int)(blockDim.x >> 6) - 1;
-  GuardBox* boxes = reinterpret_cast<GuardBox*>(reinterpret_cast<char*>(lds) + svc_box_offset(c));
+  GuardBox* boxes = reinterpret_cast<GuardBox*>(lds);
   uint32_t* done = reinterpret_cast<uint32_t*>(boxes + n_boxes);
   uint32_t* pending = done + 1;
   if (threadIdx.x == 0) {
@@ -438,8 +386,17 @@ __global__ __launch_bounds__(1024, MINW) void k_transport_svc(DevCfg c, RunArgs 
     return;
   }
   uint32_t n_events = 0, n_fp64 = 0;
-  transport_loop<MCD_MODE_DS, NCH, 3, true, false, true>(c, lds, tabs, R, n_events, n_fp64, boxes + (w - 1),
-                                                         pending);
+  LaneEl rest;
+  transport_loop<MCD_MODE_DS, NCH, 3, true, false, true, true>(c, pick, tabs, R, n_events, n_fp64, boxes + (w - 1),
+                                                               pending, &rest);
+  {
+    // The last electrons as in k_transport_f32; their windows take the place of
+    // the mailbox's slots, which are free between two posts.
+    typedef Fp32DsServed<NCH> P;
+    const KernelArgs& A = args_anew();
+    typename P::Staged* win = reinterpret_cast<typename P::Staged*>(boxes[w - 1].lane);
+    if (A.R.drain) window_drain<P>(A.c, A.R, pick, tabs, win, rest, n_events, n_fp64);
+  }
   const int lane = threadIdx.x & 63;
   // every lane is converged here; the service wavefront stops once all are counted
   if (lane == 0) __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1128,7 +1085,9 @@ static hipError_t svc_nch(const DevCfg& c, const RunArgs* R, int grid, int block
     *occ = nb < 1 ? 1 : nb;
     return hipSuccess;
   }
-  hipLaunchKernelGGL((k_transport_svc<NCH, MINW>), dim3(grid), dim3(block), lds, s, c, *R);
+  RunArgs D = *R;
+  D.drain = R->rows ? 0 : kDrain;
+  hipLaunchKernelGGL((k_transport_svc<NCH, MINW>), dim3(grid), dim3(block), lds, s, c, D);
   return hipGetLastError();
 }
 

@@ -151,8 +151,8 @@ __device__ __forceinline__ void ds_energies(const DevCfg& c, const float* __rest
 struct Fp32Base {
   typedef float Real;
   typedef F2 Energy;
-  struct alignas(16) Staged {
-    float l, ct, st, cp, sp, pad[3];
+  struct alignas(8) Staged {
+    float l, ct, st, cp, sp, pad;
   };
   struct Step {
     float l, c2, s2;
@@ -206,6 +206,7 @@ struct Fp32Base {
 template <int NCH>
 struct Fp32Ds : Fp32Base {
   static constexpr bool kPickTable = true;
+  static constexpr bool kServed = false;
   static constexpr int kTurns = 1;
   struct Draw {
     float u0, lg1, u2, az;
@@ -241,9 +242,46 @@ struct Fp32Ds : Fp32Base {
   }
 };
 
+// In the served-guard kernel: wide pick records, guard picks through the
+// wavefront's mailbox (at the start of the workgroup's LDS).
+template <int NCH>
+struct Fp32DsServed : Fp32Ds<NCH> {
+  static constexpr bool kServed = true;
+  typedef typename Fp32Ds<NCH>::Draw Draw;
+  typedef typename Fp32Ds<NCH>::Step Step;
+  typedef typename Fp32Ds<NCH>::Staged Staged;
+  static_assert(sizeof(Staged) == sizeof(GuardSlot), "a window takes the place of a mailbox's slots");
+  static __device__ __forceinline__ void step(const DevCfg& c, const float* __restrict__ lds,
+                                              const DevTable* __restrict__ tabs, F2 E, const Draw& r, Step& s) {
+    float mfp_ln2;
+    PickEval<NCH> pe;
+    s.flags = 0;
+    s.ch = f_pick_table<NCH, true>(lds, c.pick, E.hi, r.u0, mfp_ln2, pe);
+    if (__any(s.ch < 0)) {
+      extern __shared__ float lds0[];
+      const int n_boxes = (int)(blockDim.x >> 6) - 1;
+      GuardBox* boxes = reinterpret_cast<GuardBox*>(lds0);
+      served_pick<NCH>(boxes + (__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) - 1),
+                       reinterpret_cast<uint32_t*>(boxes + n_boxes) + 1, args_anew().R.guard_spins, E, r.u0, pe, s.ch,
+                       s.flags);
+    }
+    s.l = -mfp_ln2 * r.lg1;
+    ds_loss_angles(c, tabs, E, s.ch, r.u2, s.W.hi, s.W.lo, s.c2, s.s2, s.flags);
+  }
+  static __device__ __forceinline__ void energies(const DevCfg& c, const float* __restrict__ lds,
+                                                  const DevTable* __restrict__ tabs, Staged*, F2 E0,
+                                                  const Draw (&r)[1], const bool (&todo)[1], const Group& g, int,
+                                                  F2 (&Ej)[1], Step (&s)[1]) {
+    ds_energies<Fp32DsServed<NCH>>(c, lds, tabs, E0, r[0], todo[0], g, Ej[0], s[0]);
+    // the staged steps that follow overwrite the slots the picks were read from
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+};
+
 template <bool EXPL>
 struct Fp32Cont : Fp32Base {
   static constexpr bool kPickTable = false;
+  static constexpr bool kServed = false;
   static constexpr int kTurns = 4;
   struct Draw {
     float ln0, u1, az;
@@ -306,6 +344,7 @@ template <int NCH>
 struct Fp64Ds {
   typedef double Real;
   typedef double Energy;
+  static constexpr bool kServed = false;
   static constexpr bool kPickTable = false;
   static constexpr int kTurns = 1;
   struct alignas(16) Staged {
@@ -627,8 +666,10 @@ __device__ __forceinline__ void window_loop(const DevCfg& c, const RunArgs& R, c
       n_fp64 += mine && (st[i].flags & MCD_FLAG_FP64_PICK) ? 1u : 0u;
       if (__any(mine && st[i].flags)) {
 #pragma unroll
-        for (uint32_t bit = 1u; bit <= 8u; bit <<= 1)
+        for (uint32_t bit = 1u; bit <= (P::kServed ? 16u : 8u); bit <<= 1)
           if (g.ballot(mine && (st[i].flags & bit))) s.flags |= bit;
+        if (P::kServed && mine && (st[i].flags & MCD_FLAG_GUARD_TIMEOUT))
+          atomicAdd(R.counters + MCD_CNT_GUARD_TIMEOUTS, 1ull);
       }
     }
     if constexpr (ROWS) {

@@ -142,3 +142,17 @@ def test_continuous_drain_equals_one_lane_per_electron(kw, n):
     kw = dict(kw)
     tr = engine.Transport(kw.pop("material"), 10000.0, 1000.0, mode="cont", **{"s_tilt": 60.0, **kw})
     _same(tr.run(n, seed=3, first=9, block=256), tr.run(n, seed=3, first=9, waves_per_simd=5))
+
+
+# the served guard: the last electrons' windows lie in the mailboxes, their guard picks are served
+@pytest.mark.parametrize("kw", [
+    dict(),
+    dict(material="Au", E0=30000.0, Wc=20.0),
+    dict(material="Al", E0=5000.0, Emin=500.0, tilt=0.0, thickness=2000.0),
+    dict(max_scatt=65), dict(max_scatt=1),
+], ids=str)
+@pytest.mark.parametrize("n,first,shape", [(1, 0, {}), (961, 5, dict(block=128)), (40000, (1 << 32) - 60, dict(waves_per_simd=6)),
+                                           (600001, 0, {})])
+def test_ds_served_drain_equals_one_lane_per_electron(kw, n, first, shape):
+    tr = _transport(**kw)
+    _same(tr.run(n, seed=6, first=first, guard="service", **shape), tr.run(n, seed=6, first=first, waves_per_simd=5))
