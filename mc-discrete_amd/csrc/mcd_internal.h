@@ -150,7 +150,13 @@ hipError_t launch_build_tables_batched(const CdfJob* jobs, int n_jobs, long long
                                        hipStream_t s);
 hipError_t launch_pick_nodes(const DevCfg& c, int n_nodes, double lnE0, double dln, float* nodes, int stride,
                              hipStream_t s);
-hipError_t launch_pick_check(const DevCfg& c, int n_checks, float* err, int* bad, hipStream_t s);
+hipError_t launch_pick_check(const DevCfg& c, float* nodes, hipStream_t s);
+constexpr int kPickChecks = 16;  // check points per cell
+// Kept behind the last node of a pick table while it is built.
+struct PickSummary {
+  uint32_t max_err;  // bits of the largest interpolation error (not negative)
+  int n_swap, n_exact;
+};
 hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int n, hipStream_t s);
 hipError_t launch_unmask(const float* src, float* dst, size_t n, hipStream_t s);
 hipError_t launch_mask(const float* src, float* dst, size_t n, hipStream_t s);

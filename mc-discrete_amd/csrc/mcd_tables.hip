@@ -5,9 +5,10 @@
 //   trapezoids and cumulative sums (rounded to float32 once), or the float32
 //   arithmetic of the reference.  The mask W[j+1] > (E - E_F)/2 is evaluated in
 //   float32 exactly as the reference's float32 arrays do (:429-439).
-// * k_pick_nodes / k_pick_check: the LDS pick table (sorted cumulative channel
-//   probabilities and ln mfp on a ln E grid) and its interpolation-error check
-//   against the exact FP64 pick, which sets the guard band.
+// * k_pick_nodes / k_pick_cells / k_pick_check: the LDS pick table (sorted
+//   cumulative channel probabilities and ln mfp on a ln E grid), the kinds of its
+//   cells, and its interpolation-error check against the exact FP64 pick, which
+//   sets the guard band.  What the host needs of them is a PickSummary.
 #include <hip/hip_runtime.h>
 
 #include "mcd_device.h"
@@ -292,6 +293,7 @@ hipError_t launch_build_rows(const float* cdf, const float* Es, int nE, int nW, 
 
 // ---------------------------------------------------------------------------
 // pick-table nodes: FP64 sorted cumulative probabilities, ln mfp, labels.
+// The table's (zeroed) summary follows the last node.
 __global__ void k_pick_nodes(DevCfg c, int n_nodes, double lnE0, double dln, float* nodes, int stride) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n_nodes) return;
@@ -329,32 +331,61 @@ __global__ void k_pick_nodes(DevCfg c, int n_nodes, double lnE0, double dln, flo
   o[n] = __uint_as_float(lo);
   o[n + 1] = __uint_as_float(hi | (kMetaNoSwap << 12));
   for (int i = n + 2; i < stride; ++i) o[i] = 0.f;
+  if (k == 0) *reinterpret_cast<PickSummary*>(nodes + (size_t)n_nodes * stride) = PickSummary{0u, 0, 0};
+}
+
+// The kind of cell k (node k to k + 1): the same order of the channels at both
+// ends, two neighbours swapped, or exact (any other reordering, a NaN node).
+__global__ void k_pick_cells(int n_nodes, int n_ch, float* nodes, int stride) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k + 1 >= n_nodes) return;
+  float* a = nodes + (size_t)k * stride;
+  const float* b = a + stride;
+  auto label = [n_ch](const float* node, int pos) {
+    return (__float_as_uint(node[n_ch + (pos >> 3)]) >> (4 * (pos & 7))) & 15u;
+  };
+  int ndiff = 0, first = -1;
+  for (int q = 0; q < n_ch; ++q)
+    if (label(a, q) != label(b, q)) {
+      if (first < 0) first = q;
+      ++ndiff;
+    }
+  uint32_t swap = kMetaNoSwap;
+  bool exact = false;
+  if (ndiff == 2 && first + 1 < n_ch && label(a, first) == label(b, first + 1) && label(a, first + 1) == label(b, first))
+    swap = (uint32_t)first;
+  else if (ndiff != 0)
+    exact = true;
+  for (int q = 0; q < stride; ++q)
+    if (!(a[q] == a[q])) exact = true;
+  const uint32_t hi = (__float_as_uint(a[n_ch + 1]) & 0xFFFu) | (swap << 12) | (exact ? kMetaExact : 0u);
+  a[n_ch + 1] = __uint_as_float(hi);
+  PickSummary* sum = reinterpret_cast<PickSummary*>(nodes + (size_t)n_nodes * stride);
+  if (swap != kMetaNoSwap) atomicAdd(&sum->n_swap, 1);
 }
 
 hipError_t launch_pick_nodes(const DevCfg& c, int n_nodes, double lnE0, double dln, float* nodes, int stride,
                              hipStream_t s) {
   hipLaunchKernelGGL(k_pick_nodes, dim3((n_nodes + 63) / 64), dim3(64), 0, s, c, n_nodes, lnE0, dln, nodes, stride);
+  hipLaunchKernelGGL(k_pick_cells, dim3((n_nodes + 63) / 64), dim3(64), 0, s, n_nodes, c.n_shells + 3, nodes, stride);
   return hipGetLastError();
 }
 
-// Check points t = (m + 0.5)/M inside every cell: compare the FP32
+// Check points t = (m + 0.5)/16 inside every cell: compare the FP32
 // interpolation (the transport's own f_pick_eval) with the exact FP64 order and
-// cumulative probabilities.  err[2*i] = max boundary error, err[2*i+1] = error
-// of pA - pB in swap cells; bad[i] = order mismatch not explained by the swap.
+// cumulative probabilities.  err = max boundary error, err_ab = error of pA - pB
+// in swap cells; bad = order mismatch not explained by the swap.
 template <int NCH>
-__global__ void k_pick_check(DevCfg c, int M, float* err, int* bad) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void pick_point(const DevCfg& c, int k, int m, float& err, float& err_ab, bool& bad) {
   const int ncell = c.pick.n_nodes - 1;
-  if (i >= ncell * M) return;
-  const int k = i / M, m = i % M;
   const double lnE0 = log(c.Emin);
-  const double lnE = lnE0 + ((double)k + ((double)m + 0.5) / (double)M) * (log(c.E0) - lnE0) / (double)ncell;
+  const double lnE = lnE0 + ((double)k + ((double)m + 0.5) / (double)kPickChecks) * (log(c.E0) - lnE0) / (double)ncell;
   const double E = exp(lnE);
   PickEval<NCH> o;
   f_pick_eval<NCH>(c.pick.nodes, c.pick, (float)E, o);
-  err[2 * i] = 0.f;
-  err[2 * i + 1] = 0.f;
-  bad[i] = 0;
+  err = 0.f;
+  err_ab = 0.f;
+  bad = false;
   if (o.exact) return;
   double sig[MCD_MAX_CHANNELS], probs[MCD_MAX_CHANNELS];
   int lab[MCD_MAX_CHANNELS], order[MCD_MAX_CHANNELS];
@@ -385,7 +416,7 @@ __global__ void k_pick_check(DevCfg c, int M, float* err, int* bad) {
       if ((uint32_t)lab[q] == lb) sb = sig[q];
     }
     const double dtrue = (sa - sb) / s;
-    err[2 * i + 1] = fabsf((float)((double)(o.pA - o.pB) - dtrue));
+    err_ab = fabsf((float)((double)(o.pA - o.pB) - dtrue));
     if (mism) {
       // allowed only when the two orders differ by the swap itself (then the
       // guard must catch it: the boundary error at j is not meaningful)
@@ -399,22 +430,50 @@ __global__ void k_pick_check(DevCfg c, int M, float* err, int* bad) {
       eb = eb2;
     }
   }
-  err[2 * i] = eb;
-  bad[i] = mism;
+  err = eb;
+  bad = mism != 0;
 }
 
-hipError_t launch_pick_check(const DevCfg& c, int M, float* err, int* bad, hipStream_t s) {
-  const int total = (c.pick.n_nodes - 1) * M;
-  const dim3 g((total + 63) / 64), b(64);
+// 16 lanes to a cell.  A cell with a bad point, or an error that is NaN or above
+// 1e-4 (badly resolved), becomes exact; the largest error of the others is the
+// table's.
+template <int NCH>
+__global__ __launch_bounds__(64) void k_pick_check(DevCfg c, float* nodes) {
+  static_assert(kPickChecks == 16, "16 lanes share a cell");
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = i / kPickChecks, m = i % kPickChecks;
+  if (k >= c.pick.n_nodes - 1) return;
+  float err, err_ab;
+  bool bad;
+  pick_point<NCH>(c, k, m, err, err_ab, bad);
+  bad = bad || !(err == err) || !(err_ab == err_ab);
+  float ek = fmaxf(0.f, fmaxf(err, err_ab));
+#pragma unroll
+  for (int off = 1; off < kPickChecks; off <<= 1) ek = fmaxf(ek, __shfl_xor(ek, off));
+  const uint64_t any_bad = (__ballot(bad) >> ((threadIdx.x & 63) & ~(kPickChecks - 1))) & 0xFFFFull;
+  if (m) return;
+  PickSummary* sum = reinterpret_cast<PickSummary*>(nodes + (size_t)c.pick.n_nodes * c.pick.stride);
+  float* meta = nodes + (size_t)k * c.pick.stride + NCH + 1;
+  const uint32_t hi = __float_as_uint(*meta);
+  if ((hi & kMetaExact) || any_bad || (double)ek > 1e-4) {
+    *meta = __uint_as_float(hi | kMetaExact);
+    atomicAdd(&sum->n_exact, 1);
+  } else {
+    atomicMax(&sum->max_err, __float_as_uint(ek));
+  }
+}
+
+hipError_t launch_pick_check(const DevCfg& c, float* nodes, hipStream_t s) {
+  const dim3 g(((c.pick.n_nodes - 1) * kPickChecks + 63) / 64), b(64);
   switch (c.n_shells + 3) {
-    case 4: hipLaunchKernelGGL(k_pick_check<4>, g, b, 0, s, c, M, err, bad); break;
-    case 5: hipLaunchKernelGGL(k_pick_check<5>, g, b, 0, s, c, M, err, bad); break;
-    case 6: hipLaunchKernelGGL(k_pick_check<6>, g, b, 0, s, c, M, err, bad); break;
-    case 7: hipLaunchKernelGGL(k_pick_check<7>, g, b, 0, s, c, M, err, bad); break;
-    case 8: hipLaunchKernelGGL(k_pick_check<8>, g, b, 0, s, c, M, err, bad); break;
-    case 9: hipLaunchKernelGGL(k_pick_check<9>, g, b, 0, s, c, M, err, bad); break;
-    case 10: hipLaunchKernelGGL(k_pick_check<10>, g, b, 0, s, c, M, err, bad); break;
-    case 11: hipLaunchKernelGGL(k_pick_check<11>, g, b, 0, s, c, M, err, bad); break;
+    case 4: hipLaunchKernelGGL(k_pick_check<4>, g, b, 0, s, c, nodes); break;
+    case 5: hipLaunchKernelGGL(k_pick_check<5>, g, b, 0, s, c, nodes); break;
+    case 6: hipLaunchKernelGGL(k_pick_check<6>, g, b, 0, s, c, nodes); break;
+    case 7: hipLaunchKernelGGL(k_pick_check<7>, g, b, 0, s, c, nodes); break;
+    case 8: hipLaunchKernelGGL(k_pick_check<8>, g, b, 0, s, c, nodes); break;
+    case 9: hipLaunchKernelGGL(k_pick_check<9>, g, b, 0, s, c, nodes); break;
+    case 10: hipLaunchKernelGGL(k_pick_check<10>, g, b, 0, s, c, nodes); break;
+    case 11: hipLaunchKernelGGL(k_pick_check<11>, g, b, 0, s, c, nodes); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

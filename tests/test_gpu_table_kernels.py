@@ -1,5 +1,6 @@
-"""CDF rows of the loss tables (k_build_cdf: a wavefront to a row, tiles of 256
-loss bins) at the edges of its tiles, against FP64 sums in numpy."""
+"""Table kernels.  CDF rows (k_build_cdf: a wavefront to a row, tiles of 256
+loss bins) at the edges of its tiles, against FP64 sums in numpy; the kinds of the
+pick table's cells (k_pick_cells, k_pick_check)."""
 import numpy as np
 import pytest
 
@@ -53,3 +54,20 @@ def test_cdf_rows_equal_sequential_fp64_sums(nE, nW):
                 assert np.abs(got[i, :m[i]] - ref[i, :m[i]]).max(initial=0.0) <= tol, (q, prec, i)
             masked = [set(np.unique(got[i, m[i]:])) for i in range(nE)]
             assert all(len(v) <= 1 for v in masked)
+
+
+# Cell kinds and guard bands as a classification of the node orders and check errors on the host gave them
+# (swapped neighbours, exact cells at thresholds and in coarse tables); the band within float32's last digit
+@pytest.mark.parametrize("kw,nodes,swaps,exact,delta", [
+    (dict(material="Al", E0=5000.0, Emin=80.0, Wc=20.0), 16, 1, 11, 0.00017833914898801595),
+    (dict(material="Al", E0=5000.0, Emin=80.0, Wc=20.0), 512, 1, 0, 1.1658748917398043e-06),
+    (dict(material="Si", E0=3000.0, Emin=105.0, Wc=100.0, elastic="Ruth_nigram"), 17, 2, 4, 0.00015346590953413397),
+    (dict(material="Si", E0=3000.0, Emin=105.0, Wc=100.0, elastic="Ruth_nigram"), 512, 2, 11, 0.0001922775263665244),
+    (dict(material="Cu", E0=1500.0, Emin=60.0, Wc=50.0), 100, 2, 10, 0.00018746251589618623),
+    (dict(material="Au", E0=30000.0, Emin=90.0, Wc=20.0), 16, 2, 4, 0.00016507641703356057),
+    (dict(material="Au", E0=30000.0, Emin=90.0, Wc=20.0), 100, 4, 0, 1.8642254872247577e-05),
+], ids=str)
+def test_pick_table_cells_and_guard_band(kw, nodes, swaps, exact, delta):
+    info = engine.Transport(tol_E=5e-2, tol_W=5e-2, grid_search="library", pick_nodes=nodes, **kw).pick_info()
+    assert (info["n_nodes"], info["swap_cells"], info["exact_cells"]) == (nodes, swaps, exact)
+    assert abs(info["delta"] - delta) <= 2.4e-7
