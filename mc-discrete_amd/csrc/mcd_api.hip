@@ -1064,6 +1064,7 @@ static int forward_impl(mcd_ctx* ctx, const mcd_config* cfg, const mcd_tables* t
     uint64_t grid = (uint64_t)ctx->n_cu * (uint64_t)per_cu;
     if (grid > want) grid = want;
     if (grid < 1) grid = 1;
+    R.simd_waves = (int)(n / (64ull * 4 * (uint64_t)ctx->n_cu));
     HIP_TRY(ctx, launch_fill_u64(q, 0ull, 1, s));
     HIP_TRY(ctx, launch_transport(c, R, precision, minw, (int)grid, block, s));
   }

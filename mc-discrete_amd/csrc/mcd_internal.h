@@ -32,6 +32,7 @@ struct RunArgs {
   unsigned long long* park_count;    // electrons parked by the first kernel
   unsigned long long* resume_queue;  // work counter of the resume kernel
   uint32_t refill_mask;              // idle lanes are refilled every (refill_mask + 1) steps
+  int simd_waves;                    // wavefronts per SIMD a launch fills with one lane per electron
   int drain, win_off;                // last electrons of a wavefront: their number, byte offset of their windows in LDS
   uint32_t guard_spins;              // served guard: polls a transport wavefront waits for a reply
 };

@@ -115,7 +115,7 @@ __device__ void guard_service(const DevCfg& c, GuardBox* boxes, uint32_t* pendin
 // DRAIN: once the work counter is spent and at most R.drain lanes are left, the
 // loop ends and hands them over in `rest`.
 template <int MODE, int NCH, int PHASE = 0, bool PERIOD = false, bool EXPL = false, bool WIDE = false,
-          bool DRAIN = false, bool ITEM = false>
+          bool DRAIN = false, bool ITEM = false, bool PRIO = PHASE == 3>
 __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __restrict__ lds,
                                                const DevTable* __restrict__ tabs, const RunArgs& R,
                                                uint32_t& n_events, uint32_t& n_fp64, GuardBox* box = nullptr,
@@ -133,6 +133,7 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
   float p[3] = {0.f, 0.f, 0.f}, pc[3] = {0.f, 0.f, 0.f}, d[3] = {0.f, 0.f, 0.f}, y[3] = {0.f, 0.f, 0.f};
 
   uint32_t iter = 0;
+  [[maybe_unused]] uint32_t piter = 0;
   const uint32_t refill_mask = PERIOD ? R.refill_mask : 0u;
   while (true) {
     // the key words stay loop-carried SGPR values (set where all lanes are
@@ -197,12 +198,12 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
       }
     }
     if (!__any(active)) break;
-    if constexpr (PHASE == 3) {
-      // Wavefronts holding high-energy electrons (the longest remaining
-      // trajectories) issue before the others on their SIMD, so the electrons
-      // started last are not the ones left running alone after the work
-      // counter is spent (measured: 2^22-electron launch 16.1 -> 15.4 ms; the
-      // same rule applied only past the end of the counter gave 16.0 ms).
+    // Wavefronts holding high-energy electrons (the longest remaining
+    // trajectories) issue before the others on their SIMD, so the electrons
+    // started last are not the ones left running alone after the work counter
+    // is spent.  Served kernel, 2^22 electrons: 16.1 -> 15.4 ms (the same rule
+    // applied only past the end of the counter gave 16.0 ms).
+    if (PRIO && (PHASE == 3 || (piter++ & 7u) == 0u)) {
       const float span = c.E0_hi - c.Emin_hi;
       if (__any(active && E.hi > c.Emin_hi + 0.5f * span)) __builtin_amdgcn_s_setprio(3);
       else if (__any(active && E.hi > c.Emin_hi + 0.2f * span)) __builtin_amdgcn_s_setprio(2);
@@ -320,7 +321,8 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
 
 // MINW: minimum resident wavefronts per SIMD the register allocation must
 // allow (1 = compiler's choice, the default; others per launch).
-template <int MODE, int NCH, int MINW, int PHASE = 0, bool EXPL = false>
+// PRIO: issue priority by energy, every eighth step.
+template <int MODE, int NCH, int MINW, int PHASE = 0, bool EXPL = false, bool PRIO = false>
 __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R) {
   extern __shared__ float lds[];
   DevTable* tabs = nullptr;
@@ -331,8 +333,8 @@ __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R
   uint32_t n_events = 0, n_fp64 = 0;
   constexpr bool drain = PHASE == 0 && MINW == 4;
   LaneEl rest;
-  transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain>(c, lds, tabs, R, n_events, n_fp64, nullptr, nullptr,
-                                                             &rest);
+  transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain, false, PRIO>(c, lds, tabs, R, n_events, n_fp64, nullptr,
+                                                                          nullptr, &rest);
   if constexpr (drain) {
     typedef typename std::conditional<MODE == MCD_MODE_DS, Fp32Ds<NCH>, Fp32Cont<EXPL>>::type P;
     // The arguments read anew: shared with the loop above, the drain's uses
@@ -945,6 +947,17 @@ static hipError_t launch_f32(const DevCfg& c, const RunArgs& R, int grid, int bl
   RunArgs D = R;
   const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
   if (R.rows || MINW != 4) D.drain = 0;
+  // Continuous mode from three wavefronts per SIMD on, where they take turns: in
+  // us without and with the priority, 50021 electrons (JL, less than one per
+  // SIMD) 1393 and 1405, 2^19 3776 and 3307, 2^22 11186 and 10624; explicit law
+  // 2^19 5764 and 5242, 2^22 27992 and 27475.  DS steps are longer and gain
+  // less than it costs them (2^18 Cu 2873 and 2771, but 2^20 Au 12019 and 12217).
+  if constexpr (MODE == MCD_MODE_CONT && MINW == 4) {
+    if (R.simd_waves >= 3) {
+      hipLaunchKernelGGL((k_transport_f32<MODE, NCH, MINW, 0, EXPL, true>), dim3(grid), dim3(block), lds, s, c, D);
+      return hipGetLastError();
+    }
+  }
   hipLaunchKernelGGL((k_transport_f32<MODE, NCH, MINW, 0, EXPL>), dim3(grid), dim3(block), lds, s, c, D);
   return hipGetLastError();
 }

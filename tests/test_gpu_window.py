@@ -156,3 +156,11 @@ def test_continuous_drain_equals_one_lane_per_electron(kw, n):
 def test_ds_served_drain_equals_one_lane_per_electron(kw, n, first, shape):
     tr = _transport(**kw)
     _same(tr.run(n, seed=6, first=first, guard="service", **shape), tr.run(n, seed=6, first=first, waves_per_simd=5))
+
+
+# the form with issue priorities begins at three wavefronts per SIMD (196608 electrons on 256 CUs)
+@pytest.mark.parametrize("law", ["JL", "explicit"])
+@pytest.mark.parametrize("n", [196607, 196608, 262145])
+def test_continuous_priority_form_equals_the_others(law, n):
+    tr = engine.Transport("Au", 6000.0, 1000.0, s_tilt=60.0, mode="cont", bethe_model=law)
+    _same(tr.run(n, seed=3, first=9), tr.run(n, seed=3, first=9, waves_per_simd=5))
