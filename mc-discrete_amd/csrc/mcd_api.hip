@@ -1097,6 +1097,8 @@ struct mcd_batch {
   int device;
   int n_items;
   int slice_floats;
+  int default_block;
+  bool short_run;  // see batch_drains
   std::vector<mcd_tables*> own_tables;  // per-item pick tables sized for the LDS slices
   BatchItemDev* d_items;                // grouped by XCD, followed by the group bounds (n_groups + 1 ints)
   int* d_group_start;
@@ -1232,6 +1234,17 @@ extern "C" int mcd_batch_create(mcd_ctx* ctx, const mcd_batch_item* items, int n
     group_start.push_back((int)order.size());
   }
   b->slice_floats = batched_cfg_floats() + (slice > 0 ? slice : 4);
+  // Workgroups of one wavefront where LDS then holds more wavefronts per CU: with
+  // 8 KB pick tables 18 of them, and 16 in workgroups of 4 (64 configurations:
+  // 55.6 ms against 58.4, and 55.8 in workgroups of 2); equal residency keeps 4.
+  b->default_block = batched_blocks_per_cu(0, 64, b->slice_floats, false, false) >
+                             4 * batched_blocks_per_cu(0, 256, b->slice_floats, false, false) ? 64 : 256;
+  double total = 0., longest = 0.;
+  for (int i = 0; i < n_items; ++i) {
+    total += work[i];
+    if (items[i].n) longest = std::max(longest, (double)h[i].cost);
+  }
+  b->short_run = total < 10. * longest * (16. * 64. * ctx->n_cu);
   const size_t items_bytes = ((size_t)n_items * sizeof(BatchItemDev) + 255) & ~(size_t)255;
   if (hipMalloc(&b->d_items, items_bytes + (kMaxXcdGroups + 1) * sizeof(int)) != hipSuccess ||
       hipMalloc(&b->d_work, 4 * (size_t)n_items * sizeof(unsigned long long)) != hipSuccess) {
@@ -1273,27 +1286,41 @@ extern "C" int mcd_batch_create(mcd_ctx* ctx, const mcd_batch_item* items, int n
   return MCD_OK;
 }
 
+// Whether an inline run takes the form with a drain.  Runs whose work per lane
+// is less than ten of their longest trajectories end in those (ms with the
+// drain, without, and without in workgroups of one wavefront; the share of the
+// 64-configuration workload's electrons and of its configurations):
+//   1, 64    57.7 58.2 55.6     0.7, 64  43.3 43.6 41.7    0.7, 20  13.6 15.0 15.1
+//   0.1, 64  12.1 13.6 12.6     0.1, 8    6.5  8.2  9.2    0.01, 64  7.6  8.5  8.5
+// It needs 119 VGPRs, so 4 wavefronts per SIMD are the most it can keep.
+static bool batch_drains(const mcd_batch* b, int form, int block, bool period) {
+  if (form != 0 || !b->short_run) return false;
+  const int waves = block / 64;
+  return batched_blocks_per_cu(0, block, b->slice_floats, period, true) * waves >=
+         std::min(16, std::max(1, batched_blocks_per_cu(0, block, b->slice_floats, period, false) * waves));
+}
+
 // guard placement of a batch run: 0 inline, 1 deferred (phases 1 + 2), 3 served;
 // refill_mask: compaction period less one
 static hipError_t batch_enqueue(mcd_ctx* ctx, mcd_batch* b, uint64_t seed, uint64_t* counters, int form,
-                                int block, uint32_t refill_mask, hipStream_t s) {
+                                int block, bool drain, uint32_t refill_mask, hipStream_t s) {
   hipError_t e = launch_fill_u64(b->d_work, 0ull, 4 * b->n_items, s);
   unsigned long long* cnt = (unsigned long long*)counters;
   const bool deferred = form == 1;
   auto run = [&](int phase, int grid) {
     return launch_batched(b->d_items, b->n_items, b->d_group_start, b->n_groups, b->slice_floats, seed,
-                          refill_mask, cnt, phase, grid, block, s);
+                          refill_mask, cnt, phase, grid, block, phase == 0 && drain, s);
   };
   if (form == 3) {
-    const int g3 = ctx->n_cu * batched_blocks_per_cu(3, block, b->slice_floats, refill_mask != 0u);
+    const int g3 = ctx->n_cu * std::max(1, batched_blocks_per_cu(3, block, b->slice_floats, refill_mask != 0u, false));
     if (e == hipSuccess) e = run(3, g3);
   } else if (deferred) {
-    const int g1 = ctx->n_cu * batched_blocks_per_cu(1, block, b->slice_floats, refill_mask != 0u);
-    const int g2 = ctx->n_cu * batched_blocks_per_cu(2, block, b->slice_floats, false);
+    const int g1 = ctx->n_cu * std::max(1, batched_blocks_per_cu(1, block, b->slice_floats, refill_mask != 0u, false));
+    const int g2 = ctx->n_cu * std::max(1, batched_blocks_per_cu(2, block, b->slice_floats, false, false));
     if (e == hipSuccess) e = run(1, g1);
     if (e == hipSuccess) e = run(2, g2);
   } else {
-    const int g0 = ctx->n_cu * batched_blocks_per_cu(0, block, b->slice_floats, refill_mask != 0u);
+    const int g0 = ctx->n_cu * std::max(1, batched_blocks_per_cu(0, block, b->slice_floats, refill_mask != 0u, drain));
     if (e == hipSuccess) e = run(0, g0);
   }
   if (e == hipSuccess) e = launch_count_outcomes_batched(b->d_items, b->n_items, cnt, s);
@@ -1315,17 +1342,20 @@ extern "C" int mcd_batch_run(mcd_ctx* ctx, mcd_batch* b, uint64_t seed, uint64_t
   // electrons (its service wavefronts then stay idle), the deferred form then
   // runs as the inline one
   const int form = (flags & MCD_LAUNCH_SERVICE_GUARD) ? 3 : ((b->has_ds && (flags & MCD_LAUNCH_DEFER_GUARD)) ? 1 : 0);
-  const int block = launch && launch->block > 0 ? launch->block : 256;
+  const bool given = launch && launch->block > 0;
+  const uint32_t refill = (1u << ((flags & MCD_LAUNCH_REFILL_MASK) >> MCD_LAUNCH_REFILL_SHIFT)) - 1u;
+  int block = given ? launch->block : 256;
+  const bool drain = block % 64 == 0 && block <= 256 && batch_drains(b, form, block, refill != 0u);
+  if (!given && !drain && form != 3) block = b->default_block;
   if (form == 3) {
     if (block % 64 || block < 128 || block > 1024)
       return set_err(ctx, MCD_ERR_INVALID, "served guard: block %d must be a multiple of 64 in [128, 1024]", block);
   } else if (block % 64 || block > 256) {
     return set_err(ctx, MCD_ERR_INVALID, "block %d invalid", block);
   }
-  const uint32_t refill = (1u << ((flags & MCD_LAUNCH_REFILL_MASK) >> MCD_LAUNCH_REFILL_SHIFT)) - 1u;
   hipStream_t s = (hipStream_t)stream;
   if (!use_graph) {
-    HIP_TRY(ctx, batch_enqueue(ctx, b, seed, counters, form, block, refill, s));
+    HIP_TRY(ctx, batch_enqueue(ctx, b, seed, counters, form, block, drain, refill, s));
     return MCD_OK;
   }
   if (!b->graph || b->graph_seed != seed || b->graph_counters != counters || b->graph_block != block ||
@@ -1333,7 +1363,7 @@ extern "C" int mcd_batch_run(mcd_ctx* ctx, mcd_batch* b, uint64_t seed, uint64_t
     if (b->graph) { (void)hipGraphExecDestroy(b->graph); b->graph = nullptr; }
     if (!b->capture_stream) HIP_TRY(ctx, hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
     HIP_TRY(ctx, hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal));
-    hipError_t e = batch_enqueue(ctx, b, seed, counters, form, block, refill, b->capture_stream);
+    hipError_t e = batch_enqueue(ctx, b, seed, counters, form, block, drain, refill, b->capture_stream);
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(b->capture_stream, &g);
     HIP_TRY(ctx, e);

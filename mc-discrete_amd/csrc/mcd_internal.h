@@ -61,8 +61,9 @@ constexpr int kMaxXcdGroups = 16;
 
 hipError_t launch_batched(const BatchItemDev* items, int n_items, const int* group_start, int n_groups,
                           int slice_floats, uint64_t seed, uint32_t refill_mask, unsigned long long* counters,
-                          int phase, int grid, int block, hipStream_t s);
-int batched_blocks_per_cu(int phase, int block, int slice_floats, bool period);
+                          int phase, int grid, int block, bool drain, hipStream_t s);
+// 0 where a workgroup does not fit
+int batched_blocks_per_cu(int phase, int block, int slice_floats, bool period, bool drain);
 int batched_cfg_floats();
 
 

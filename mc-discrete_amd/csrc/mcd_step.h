@@ -26,11 +26,12 @@ __device__ __forceinline__ const KernelArgs& args_anew() {
   asm volatile("" : "+s"(p));
   return (const KernelArgs&)*p;
 }
-// A configuration in the constant address space (a batch item's).
-__device__ __forceinline__ const DevCfg& cfg_anew(const DevCfg& c) {
-  Const4<DevCfg>* p = (Const4<DevCfg>*)&c;
+// The same for an object in the constant address space (a batch item's).
+template <class T>
+__device__ __forceinline__ const T& anew(const T& x) {
+  Const4<T>* p = (Const4<T>*)&x;
   asm volatile("" : "+s"(p));
-  return (const DevCfg&)*p;
+  return (const T&)*p;
 }
 
 // LDS of the one-configuration kernels: the pick table (nf floats), then the

@@ -55,6 +55,13 @@ __device__ __forceinline__ void count_outcome_words(const mcd_electron_rec* __re
 }
 
 // ---------------------------------------------------------------------------
+// Electrons a wavefront goes on with in the window form once the work counter is
+// spent (one group of 4 lanes each).  Their last 1000 to 5000 steps cost 1.4 to
+// 1.9 us each with one lane per electron.  Launches of 2^20 electrons in us
+// without it and at 8 and 16: @@
+constexpr int kDrain = 16;
+
+// ---------------------------------------------------------------------------
 // The service wavefront's loop: answer posted mailboxes until every transport
 // wavefront of the workgroup has finished (each adds one to *done on exit;
 // a wavefront exits only after its last reply, so none is left waiting).
@@ -256,7 +263,7 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
         if (ch < 0) {  // guard band: settle the pick in FP64
           uint32_t plo, phi;
           guard_perm<NCH>(pe, plo, phi);
-          const DevCfg& ca = ITEM ? cfg_anew(c) : args_anew().c;
+          const DevCfg& ca = ITEM ? anew(c) : args_anew().c;
           ch = d_pick_ordered<NCH>((double)E.hi + (double)E.lo, (double)u0, ca, plo, phi, pe.swap, pe.exact);
           sflags |= MCD_FLAG_FP64_PICK;
           n_fp64++;
@@ -471,24 +478,38 @@ __device__ __forceinline__ int xcc_id() {
 constexpr int kCfgFloats = (int)((sizeof(DevCfg) + 15) / 16 * 4);
 
 int batched_cfg_floats() { return kCfgFloats; }
+// before them (DRAIN) the staged steps of its last electrons, which are read one past the end
+constexpr int kItemWinFloats = (int)(64 * sizeof(Fp32Base::Staged) / sizeof(float));
+constexpr int kItemTabFloats = (int)((2 * sizeof(DevTable) + 15) / 16 * 4);
 
 // PERIOD: idle lanes take new electrons every refill_mask + 1 steps (the
 // launch's compaction period), and at once when all are idle; otherwise every
 // step.  A separate instantiation, so the every-step kernels keep their
 // register budget.  c: the item's constants (scalar loads); cl: the
 // wavefront's LDS copy, whose two table descriptors the lanes select from.
-template <int MODE, int NCH, int PHASE, bool PERIOD, bool EXPL = false>
-__device__ __forceinline__ void run_item(const DevCfg& c, const DevCfg& cl, const RunArgs& itR, const float* pick,
-                                         uint64_t seed, uint32_t refill_mask, unsigned long long* ic, uint32_t& ne,
-                                         uint32_t& nf, GuardBox* box, uint32_t* pending) {
+// DRAIN: the item's last electrons as in k_transport_f32, their staged steps at
+// win (drain of them at most).
+template <int MODE, int NCH, int PHASE, bool PERIOD, bool DRAIN, bool EXPL = false>
+__device__ __forceinline__ void run_item(const DevCfg& c, const DevTable* tabs, const RunArgs& itR, const float* pick,
+                                         Fp32Base::Staged* win, uint64_t seed, uint32_t refill_mask,
+                                         unsigned long long* ic, uint32_t& ne, uint32_t& nf, GuardBox* box,
+                                         uint32_t* pending) {
   RunArgs R = itR;
   R.seed = seed;
   R.refill_mask = refill_mask;
   // the item's counter block of this launch: phases 2 and 3 count errors in it
   if constexpr (PHASE >= 2) R.counters = ic;
   // the table descriptors from the LDS copy: the per-lane Moller / Gryzinski select reads LDS
-  transport_loop<MODE, NCH, MODE == MCD_MODE_DS ? PHASE : 0, PERIOD, EXPL, false, false, true>(
-      c, pick, &cl.tm, R, ne, nf, box, pending);
+  R.drain = DRAIN ? kDrain : 0;
+  LaneEl rest;
+  transport_loop<MODE, NCH, MODE == MCD_MODE_DS ? PHASE : 0, PERIOD, EXPL, false, DRAIN, true>(
+      c, pick, tabs, R, ne, nf, box, pending, &rest);
+  if constexpr (DRAIN) {
+    typedef typename std::conditional<MODE == MCD_MODE_DS, Fp32DsItem<NCH>, Fp32Cont<EXPL>>::type P;
+    RunArgs D = anew(itR);
+    D.seed = seed;
+    window_drain<P>(anew(c), D, pick, tabs, win, rest, ne, nf);
+  }
 }
 
 // The batched kernel's service wavefront: as guard_service, for mailboxes
@@ -562,8 +583,10 @@ static size_t batched_lds_bytes(int phase, int block, int slice_floats) {
 // resident wavefronts per SIMD for phases 0, 1 and 3 (phase 0 spills at its
 // refill, FP64-guard and item-switch code and still beats 4 and 6
 // wavefronts), 4 for phase 2.
-template <int PHASE, bool PERIOD>
-__global__ __launch_bounds__(PHASE == 3 ? 1024 : 256, PHASE == 2 ? 4 : 5) void k_transport_batched(
+// DRAIN (phase 0, short runs): every item's last electrons with several lanes
+// each, 4 wavefronts per SIMD (119 VGPRs; 111 spills at 5).
+template <int PHASE, bool PERIOD, bool DRAIN = false>
+__global__ __launch_bounds__(PHASE == 3 ? 1024 : 256, PHASE == 2 || DRAIN ? 4 : 5) void k_transport_batched(
     const __attribute__((address_space(4))) BatchItemDev* __restrict__ citems, int n_items,
     const int* __restrict__ group_start, int n_groups, int slice_floats, uint64_t seed, uint32_t refill_mask,
     unsigned long long* __restrict__ counters) {
@@ -571,8 +594,10 @@ __global__ __launch_bounds__(PHASE == 3 ? 1024 : 256, PHASE == 2 ? 4 : 5) void k
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  float* my = lds + (size_t)wib * slice_floats;
-  float* pick = my + kCfgFloats;
+  float* my = lds + (size_t)wib * slice_floats + (DRAIN ? kItemWinFloats : 0);
+  float* pick = my + (DRAIN ? kItemTabFloats : kCfgFloats);
+  const DevTable* tabs = DRAIN ? reinterpret_cast<const DevTable*>(my) : &reinterpret_cast<const DevCfg*>(my)->tm;
+  Fp32Base::Staged* win = DRAIN ? reinterpret_cast<Fp32Base::Staged*>(my - kItemWinFloats) : nullptr;
   GuardBox* boxes = nullptr;
   uint32_t *done = nullptr, *pending = nullptr;
   if constexpr (PHASE == 3) {
@@ -618,8 +643,8 @@ __global__ __launch_bounds__(PHASE == 3 ? 1024 : 256, PHASE == 2 ? 4 : 5) void k
     const BatchItemDev& it = items[ci];
     if (lane == 0) atomicAdd(it.active, 1ull);
     // stage the configuration and its pick table in this wavefront's slice
-    const float* src = reinterpret_cast<const float*>(&it.c);
-    for (int i = lane; i < (int)(sizeof(DevCfg) / 4); i += 64) my[i] = src[i];
+    const float* src = DRAIN ? reinterpret_cast<const float*>(&it.c.tm) : reinterpret_cast<const float*>(&it.c);
+    for (int i = lane; i < (int)((DRAIN ? 2 * sizeof(DevTable) : sizeof(DevCfg)) / 4); i += 64) my[i] = src[i];
     const int mode = it.c.mode;
     const int nch = it.c.n_shells + 3;
     if (mode == MCD_MODE_DS) {
@@ -630,26 +655,27 @@ __global__ __launch_bounds__(PHASE == 3 ? 1024 : 256, PHASE == 2 ? 4 : 5) void k
     __builtin_amdgcn_wave_barrier();
     const DevCfg& c = *reinterpret_cast<const DevCfg*>(my);
     const DevCfg& cg = (const DevCfg&)citems[ci].c;  // the same constants as scalar loads
+    const RunArgs& rg = (const RunArgs&)citems[ci].R;
     // set only where the loop uses it, so it is not live across the other phases' loops
     unsigned long long* icl = PHASE >= 2 ? counters + (size_t)it.slot * MCD_NCOUNTERS : nullptr;
     uint32_t ne = 0, nf = 0;
     if (mode == MCD_MODE_CONT) {
       if (PHASE != 2) {
-        if (c.bethe == MCD_BETHE_EXPLICIT)
-          run_item<MCD_MODE_CONT, 4, PHASE, PERIOD, true>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, nullptr, nullptr);
+        if ((DRAIN ? cg.bethe : c.bethe) == MCD_BETHE_EXPLICIT)
+          run_item<MCD_MODE_CONT, 4, PHASE, PERIOD, DRAIN, true>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, nullptr, nullptr);
         else
-          run_item<MCD_MODE_CONT, 4, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, nullptr, nullptr);
+          run_item<MCD_MODE_CONT, 4, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, nullptr, nullptr);
       }
     } else {
       switch (nch) {
-        case 4: run_item<MCD_MODE_DS, 4, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
-        case 5: run_item<MCD_MODE_DS, 5, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
-        case 6: run_item<MCD_MODE_DS, 6, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
-        case 7: run_item<MCD_MODE_DS, 7, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
-        case 8: run_item<MCD_MODE_DS, 8, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
-        case 9: run_item<MCD_MODE_DS, 9, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
-        case 10: run_item<MCD_MODE_DS, 10, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
-        default: run_item<MCD_MODE_DS, 11, PHASE, PERIOD>(cg, c, it.R, pick, seed, refill_mask, icl, ne, nf, box, pending); break;
+        case 4: run_item<MCD_MODE_DS, 4, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
+        case 5: run_item<MCD_MODE_DS, 5, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
+        case 6: run_item<MCD_MODE_DS, 6, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
+        case 7: run_item<MCD_MODE_DS, 7, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
+        case 8: run_item<MCD_MODE_DS, 8, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
+        case 9: run_item<MCD_MODE_DS, 9, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
+        case 10: run_item<MCD_MODE_DS, 10, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
+        default: run_item<MCD_MODE_DS, 11, PHASE, PERIOD, DRAIN>(cg, tabs, rg, pick, win, seed, refill_mask, icl, ne, nf, box, pending); break;
       }
     }
     const uint64_t cnt[2] = {ne, nf};
@@ -666,14 +692,15 @@ __global__ __launch_bounds__(PHASE == 3 ? 1024 : 256, PHASE == 2 ? 4 : 5) void k
   }
 }
 
-template <int PHASE, bool PERIOD>
+template <int PHASE, bool PERIOD, bool DRAIN = false>
 static const void* batched_kernel() {
-  return reinterpret_cast<const void*>(&k_transport_batched<PHASE, PERIOD>);
+  return reinterpret_cast<const void*>(&k_transport_batched<PHASE, PERIOD, DRAIN>);
 }
 
 // The kernel of a phase; the phases that take new electrons (0, 1, 3) have a
 // compaction-period form, the resume phase (2) refills every step.
-static const void* batched_kernel(int phase, bool period) {
+static const void* batched_kernel(int phase, bool period, bool drain) {
+  if (drain) return period ? batched_kernel<0, true, true>() : batched_kernel<0, false, true>();
   switch (phase) {
     case 1: return period ? batched_kernel<1, true>() : batched_kernel<1, false>();
     case 2: return batched_kernel<2, false>();
@@ -682,24 +709,29 @@ static const void* batched_kernel(int phase, bool period) {
   }
 }
 
-hipError_t launch_batched(const BatchItemDev* items, int n_items, const int* group_start, int n_groups,
-                          int slice_floats, uint64_t seed, uint32_t refill_mask, unsigned long long* counters,
-                          int phase, int grid, int block, hipStream_t s) {
-  if (phase == 3 && (block < 128 || block > 1024)) return hipErrorInvalidValue;
-  if (n_groups < 1 || n_groups > kMaxXcdGroups) return hipErrorInvalidValue;
-  const size_t lds = batched_lds_bytes(phase, block, slice_floats);
-  const void* k = batched_kernel(phase, refill_mask != 0u);
-  void* args[] = {(void*)&items, (void*)&n_items, (void*)&group_start, (void*)&n_groups, (void*)&slice_floats,
-                  (void*)&seed, (void*)&refill_mask, (void*)&counters};
-  return hipLaunchKernel(k, dim3(grid), dim3(block), args, lds, s);
+// A slice (slice_floats without a drain) as the kernel lays it out.
+static int batched_slice(int slice_floats, bool drain) {
+  return drain ? slice_floats - kCfgFloats + kItemTabFloats + kItemWinFloats : slice_floats;
+}
+int batched_blocks_per_cu(int phase, int block, int slice_floats, bool period, bool drain) {
+  int nb = 0;
+  const size_t lds = batched_lds_bytes(phase, block, batched_slice(slice_floats, drain));
+  const void* k = batched_kernel(phase, period, drain);
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, block, lds) != hipSuccess) return 0;
+  return nb;
 }
 
-int batched_blocks_per_cu(int phase, int block, int slice_floats, bool period) {
-  int nb = 0;
-  const size_t lds = batched_lds_bytes(phase, block, slice_floats);
-  const void* k = batched_kernel(phase, period);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, block, lds) != hipSuccess || nb < 1) nb = 1;
-  return nb;
+hipError_t launch_batched(const BatchItemDev* items, int n_items, const int* group_start, int n_groups,
+                          int slice_floats, uint64_t seed, uint32_t refill_mask, unsigned long long* counters,
+                          int phase, int grid, int block, bool drain, hipStream_t s) {
+  if (phase == 3 && (block < 128 || block > 1024)) return hipErrorInvalidValue;
+  if (n_groups < 1 || n_groups > kMaxXcdGroups || (drain && phase)) return hipErrorInvalidValue;
+  int slice = batched_slice(slice_floats, drain);
+  const size_t lds = batched_lds_bytes(phase, block, slice);
+  const void* k = batched_kernel(phase, refill_mask != 0u, drain);
+  void* args[] = {(void*)&items, (void*)&n_items, (void*)&group_start, (void*)&n_groups, (void*)&slice,
+                  (void*)&seed, (void*)&refill_mask, (void*)&counters};
+  return hipLaunchKernel(k, dim3(grid), dim3(block), args, lds, s);
 }
 
 __global__ __launch_bounds__(256) void k_count_outcomes_batched(const BatchItemDev* __restrict__ items,
@@ -922,12 +954,6 @@ hipError_t launch_order_scatter(const mcd_scatter_rec* rows, uint64_t n, const m
 
 // ---------------------------------------------------------------------------
 // host-side launchers
-
-// Electrons a wavefront goes on with in the window form once the work counter is
-// spent (one group of 4 lanes each).  Their last 1000 to 5000 steps cost 1.4 to
-// 1.9 us each with one lane per electron.  Launches of 2^20 electrons in us
-// without it and at 8 and 16: @@
-constexpr int kDrain = 16;
 
 // LDS of a one-kernel launch that needs `used` bytes for its step, with the
 // windows of its last electrons after them (D.win_off, D.drain); without them

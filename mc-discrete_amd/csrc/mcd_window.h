@@ -220,6 +220,12 @@ struct Fp32Ds : Fp32Base {
   }
   static __device__ __forceinline__ void step(const DevCfg& c, const float* __restrict__ lds,
                                               const DevTable* __restrict__ tabs, F2 E, const Draw& r, Step& s) {
+    step_of<false>(c, lds, tabs, E, r, s);
+  }
+  // ITEM: as in transport_loop
+  template <bool ITEM>
+  static __device__ __forceinline__ void step_of(const DevCfg& c, const float* __restrict__ lds,
+                                                 const DevTable* __restrict__ tabs, F2 E, const Draw& r, Step& s) {
     float mfp_ln2;
     PickEval<NCH> pe;
     s.flags = 0;
@@ -227,8 +233,8 @@ struct Fp32Ds : Fp32Base {
     if (s.ch < 0) {  // guard band: settle the pick in FP64
       uint32_t plo, phi;
       guard_perm<NCH>(pe, plo, phi);
-      s.ch = d_pick_ordered<NCH>((double)E.hi + (double)E.lo, (double)r.u0, args_anew().c, plo, phi, pe.swap,
-                                  pe.exact);
+      const DevCfg& ca = ITEM ? anew(c) : args_anew().c;
+      s.ch = d_pick_ordered<NCH>((double)E.hi + (double)E.lo, (double)r.u0, ca, plo, phi, pe.swap, pe.exact);
       s.flags |= MCD_FLAG_FP64_PICK;
     }
     s.l = -mfp_ln2 * r.lg1;
@@ -239,6 +245,24 @@ struct Fp32Ds : Fp32Base {
                                                   const Draw (&r)[1], const bool (&todo)[1], const Group& g, int,
                                                   F2 (&Ej)[1], Step (&s)[1]) {
     ds_energies<Fp32Ds<NCH>>(c, lds, tabs, E0, r[0], todo[0], g, Ej[0], s[0]);
+  }
+};
+
+// A batch item's.
+template <int NCH>
+struct Fp32DsItem : Fp32Ds<NCH> {
+  typedef typename Fp32Ds<NCH>::Draw Draw;
+  typedef typename Fp32Ds<NCH>::Step Step;
+  typedef typename Fp32Ds<NCH>::Staged Staged;
+  static __device__ __forceinline__ void step(const DevCfg& c, const float* __restrict__ lds,
+                                              const DevTable* __restrict__ tabs, F2 E, const Draw& r, Step& s) {
+    Fp32Ds<NCH>::template step_of<true>(c, lds, tabs, E, r, s);
+  }
+  static __device__ __forceinline__ void energies(const DevCfg& c, const float* __restrict__ lds,
+                                                  const DevTable* __restrict__ tabs, Staged*, F2 E0,
+                                                  const Draw (&r)[1], const bool (&todo)[1], const Group& g, int,
+                                                  F2 (&Ej)[1], Step (&s)[1]) {
+    ds_energies<Fp32DsItem<NCH>>(c, lds, tabs, E0, r[0], todo[0], g, Ej[0], s[0]);
   }
 };
 
