@@ -182,8 +182,10 @@ __device__ __forceinline__ void ds_loss_angles(const DevCfg& c, const DevTable* 
 
 // Free path l, loss Wh + Wl and Joy's screening parameter a (the polar angle's)
 // of a continuous-mode step; ln_u0 = ln of the path's random number.  EXPL:
-// the explicit Bethe law, evaluated in FP64.
-template <bool EXPL>
+// the explicit Bethe law, evaluated in FP64.  NIGRAM: the screening, where the
+// caller has branched on it.
+enum { kScreenAny = -1 };
+template <bool EXPL, int NIGRAM = kScreenAny>
 __device__ __forceinline__ void cont_path_loss(const DevCfg& c, F2 E, float ln_u0, float& a, float& l, float& Wh,
                                                float& Wl, uint32_t& sflags) {
   Wl = 0.f;
@@ -191,7 +193,7 @@ __device__ __forceinline__ void cont_path_loss(const DevCfg& c, F2 E, float ln_u
   // Joy's screening: the polar angle (Rutherford_halfPol) in every model
   a = c.c_alpha_f * __builtin_amdgcn_rcpf(E.hi);
   float sig;
-  if (c.elastic >= MCD_ELASTIC_NIGRAM) {  // ruther_N_sigma(_wDefl), crossSections.py:91-147
+  if (NIGRAM == kScreenAny ? c.elastic >= MCD_ELASTIC_NIGRAM : NIGRAM) {  // ruther_N_sigma(_wDefl), crossSections.py:91-147
     const float b = 0.48f * (c.nig_zp_f * __builtin_amdgcn_rcpf(E.hi));
     sig = c.nig_num_f * __builtin_amdgcn_rcpf(4.f * b * (1.f + b) * (E.hi * E.hi));
   } else {

@@ -122,7 +122,7 @@ __device__ void guard_service(const DevCfg& c, GuardBox* boxes, uint32_t* pendin
 // DRAIN: once the work counter is spent and at most R.drain lanes are left, the
 // loop ends and hands them over in `rest`.
 template <int MODE, int NCH, int PHASE = 0, bool PERIOD = false, bool EXPL = false, bool WIDE = false,
-          bool DRAIN = false, bool ITEM = false, bool PRIO = PHASE == 3>
+          bool DRAIN = false, bool ITEM = false, bool PRIO = PHASE == 3, int NIGRAM = kScreenAny>
 __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __restrict__ lds,
                                                const DevTable* __restrict__ tabs, const RunArgs& R,
                                                uint32_t& n_events, uint32_t& n_fp64, GuardBox* box = nullptr,
@@ -275,7 +275,7 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
       const float u0 = u01f(r.x), u1 = u01f(r.y);
       u_az = u01f(r.z);
       float a;
-      cont_path_loss<EXPL>(c, E, ln_f(u0), a, l, Wh, Wl, sflags);
+      cont_path_loss<EXPL, NIGRAM>(c, E, ln_f(u0), a, l, Wh, Wl, sflags);
       const float om = 1.f - u1;
       const float inv = __builtin_amdgcn_rcpf(om + a);
       s2 = a * u1 * inv;
@@ -328,8 +328,9 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
 
 // MINW: minimum resident wavefronts per SIMD the register allocation must
 // allow (1 = compiler's choice, the default; others per launch).
-// PRIO: issue priority by energy, every eighth step.
-template <int MODE, int NCH, int MINW, int PHASE = 0, bool EXPL = false, bool PRIO = false>
+// PRIO: issue priority by energy, every eighth step.  NIGRAM (continuous mode):
+// the elastic screening, branched on at the launch instead of at every step.
+template <int MODE, int NCH, int MINW, int PHASE = 0, bool EXPL = false, bool PRIO = false, int NIGRAM = kScreenAny>
 __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R) {
   extern __shared__ float lds[];
   DevTable* tabs = nullptr;
@@ -340,8 +341,8 @@ __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R
   uint32_t n_events = 0, n_fp64 = 0;
   constexpr bool drain = PHASE == 0 && MINW == 4;
   LaneEl rest;
-  transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain, false, PRIO>(c, lds, tabs, R, n_events, n_fp64, nullptr,
-                                                                          nullptr, &rest);
+  transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain, false, PRIO, NIGRAM>(c, lds, tabs, R, n_events, n_fp64,
+                                                                                  nullptr, nullptr, &rest);
   if constexpr (drain) {
     typedef typename std::conditional<MODE == MCD_MODE_DS, Fp32Ds<NCH>, Fp32Cont<EXPL>>::type P;
     // The arguments read anew: shared with the loop above, the drain's uses
@@ -968,32 +969,39 @@ static size_t with_drain(size_t used, int block, RunArgs& D) {
   return fits ? all : used;
 }
 
+// The kernel of a launch.  Continuous mode at 4 wavefronts per SIMD: one per
+// screening, and from three wavefronts per SIMD on, where they take turns, with
+// issue priorities: in us without and with them, 50021 electrons (JL, less than
+// one per SIMD) 1393 and 1405, 2^19 3776 and 3307, 2^22 11186 and 10624; explicit
+// law 2^19 5764 and 5242, 2^22 27992 and 27475.  DS steps are longer and gain
+// less than it costs them (2^18 Cu 2873 and 2771, but 2^20 Au 12019 and 12217).
+template <int MODE, int NCH, int MINW, bool EXPL>
+static const void* f32_kernel(const DevCfg& c, int simd_waves) {
+  if constexpr (MODE == MCD_MODE_CONT && MINW == 4) {
+    if (c.elastic >= MCD_ELASTIC_NIGRAM)
+      return simd_waves >= 3 ? reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, true, 1>)
+                             : reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, false, 1>);
+    return simd_waves >= 3 ? reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, true, 0>)
+                           : reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, false, 0>);
+  }
+  return reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL>);
+}
+
 template <int MODE, int NCH, int MINW, bool EXPL>
 static hipError_t launch_f32(const DevCfg& c, const RunArgs& R, int grid, int block, size_t used, hipStream_t s) {
   RunArgs D = R;
   const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
   if (R.rows || MINW != 4) D.drain = 0;
-  // Continuous mode from three wavefronts per SIMD on, where they take turns: in
-  // us without and with the priority, 50021 electrons (JL, less than one per
-  // SIMD) 1393 and 1405, 2^19 3776 and 3307, 2^22 11186 and 10624; explicit law
-  // 2^19 5764 and 5242, 2^22 27992 and 27475.  DS steps are longer and gain
-  // less than it costs them (2^18 Cu 2873 and 2771, but 2^20 Au 12019 and 12217).
-  if constexpr (MODE == MCD_MODE_CONT && MINW == 4) {
-    if (R.simd_waves >= 3) {
-      hipLaunchKernelGGL((k_transport_f32<MODE, NCH, MINW, 0, EXPL, true>), dim3(grid), dim3(block), lds, s, c, D);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((k_transport_f32<MODE, NCH, MINW, 0, EXPL>), dim3(grid), dim3(block), lds, s, c, D);
-  return hipGetLastError();
+  void* args[] = {(void*)&c, (void*)&D};
+  return hipLaunchKernel(f32_kernel<MODE, NCH, MINW, EXPL>(c, R.simd_waves), dim3(grid), dim3(block), args, lds, s);
 }
 
 template <int MODE, int NCH, int MINW, bool EXPL>
-static int occ_f32(int block, size_t used) {
+static int occ_f32(const DevCfg& c, int block, size_t used) {
   int nb = 0;
   RunArgs D;
   const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_transport_f32<MODE, NCH, MINW, 0, EXPL>, block, lds) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f32_kernel<MODE, NCH, MINW, EXPL>(c, 0), block, lds) !=
       hipSuccess)
     return 1;
   return nb < 1 ? 1 : nb;
@@ -1006,7 +1014,7 @@ static hipError_t dispatch_w(int minw, const DevCfg& c, const RunArgs* R, int gr
   switch (minw) {
 #define MCD_W(W)                                                   \
   case W:                                                          \
-    if (occ) { *occ = occ_f32<MODE, NCH, W, EXPL>(block, lds); return hipSuccess; } \
+    if (occ) { *occ = occ_f32<MODE, NCH, W, EXPL>(c, block, lds); return hipSuccess; } \
     return launch_f32<MODE, NCH, W, EXPL>(c, *R, grid, block, lds, s);
     MCD_W(1) MCD_W(4) MCD_W(5) MCD_W(6) MCD_W(8)
 #undef MCD_W

@@ -315,6 +315,28 @@ struct Fp32Cont : Fp32Base {
   static __device__ __forceinline__ void stage(Staged& w, const Step& s, const Draw& r) {
     Fp32Base::stage(w, s, r.az);
   }
+  template <int M, int NIGRAM>
+  static __device__ __forceinline__ void chain(const DevCfg& c, const Staged* wp, F2 E0, const Group& g, int turns,
+                                               F2 (&Ej)[M]) {
+    F2 cur = E0;
+    float a, l, ln0 = wp[0].l;
+    uint32_t flags = 0;
+    int k = 0;
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      Ej[i] = cur;
+      if (i < turns) {
+        for (int kk = 0; kk < g.G; ++kk) {
+          Ej[i] = select(g.j == kk, cur, Ej[i]);
+          const float next = wp[++k].l;
+          F2 W;
+          cont_path_loss<EXPL, NIGRAM>(c, cur, ln0, a, l, W.hi, W.lo, flags);
+          cur = minus(cur, W);
+          ln0 = next;
+        }
+      }
+    }
+  }
   // Step after step: all lanes of a group form step k's loss from its staged
   // logarithm, the lane of step k keeps the energy it starts from; then every
   // lane its own steps' paths, losses and angles.
@@ -329,28 +351,14 @@ struct Fp32Cont : Fp32Base {
       if (i < turns) wp[i * g.G + g.j].l = r[i].ln0;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    F2 cur = E0;
-    float a, l, ln0 = wp[0].l;
-    uint32_t flags = 0;
-    int k = 0;
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-      Ej[i] = cur;
-      if (i < turns) {
-        for (int kk = 0; kk < g.G; ++kk) {
-          Ej[i] = select(g.j == kk, cur, Ej[i]);
-          const float next = wp[++k].l;
-          F2 W;
-          cont_path_loss<EXPL>(c, cur, ln0, a, l, W.hi, W.lo, flags);
-          cur = minus(cur, W);
-          ln0 = next;
-        }
-      }
-    }
+    // one loop per screening: a branch in it costs six instructions a step
+    if (c.elastic >= MCD_ELASTIC_NIGRAM) chain<M, 1>(c, wp, E0, g, turns, Ej);
+    else chain<M, 0>(c, wp, E0, g, turns, Ej);
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int i = 0; i < M; ++i) {
       if (!todo[i]) continue;
+      float a;
       s[i].flags = 0;
       cont_path_loss<EXPL>(c, Ej[i], r[i].ln0, a, s[i].l, s[i].W.hi, s[i].W.lo, s[i].flags);
       const float om = 1.f - r[i].u1;

@@ -164,3 +164,11 @@ def test_ds_served_drain_equals_one_lane_per_electron(kw, n, first, shape):
 def test_continuous_priority_form_equals_the_others(law, n):
     tr = engine.Transport("Au", 6000.0, 1000.0, s_tilt=60.0, mode="cont", bethe_model=law)
     _same(tr.run(n, seed=3, first=9), tr.run(n, seed=3, first=9, waves_per_simd=5))
+
+
+# quads to 3.25 wavefronts per SIMD (53248 electrons on 256 CUs), a kernel per screening on either side
+@pytest.mark.parametrize("elastic", ["Ruth_vanilla", "Ruth_nigram"])
+@pytest.mark.parametrize("law,n", [("JL", 53248), ("classical", 53249), ("JL", 196608), ("explicit", 16385)])
+def test_continuous_screenings_equal_the_general_form(elastic, law, n):
+    tr = engine.Transport("Au", 6000.0, 1000.0, s_tilt=60.0, mode="cont", bethe_model=law, elastic=elastic)
+    _same(tr.run(n, seed=5, first=2), tr.run(n, seed=5, first=2, waves_per_simd=5))
