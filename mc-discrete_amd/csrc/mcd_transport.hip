@@ -119,16 +119,19 @@ __device__ void guard_service(const DevCfg& c, GuardBox* boxes, uint32_t* pendin
 // service wavefront through `box`; same records as phase 0.
 // EXPL (continuous mode): the explicit Bethe law, evaluated in FP64.
 // ITEM: c is a batch item's configuration, not the kernel's argument.
+// ROWS: the launch may store scatter rows.
 // DRAIN: once the work counter is spent and at most R.drain lanes are left, the
 // loop ends and hands them over in `rest`.
 template <int MODE, int NCH, int PHASE = 0, bool PERIOD = false, bool EXPL = false, bool WIDE = false,
-          bool DRAIN = false, bool ITEM = false, bool PRIO = PHASE == 3, int NIGRAM = kScreenAny>
+          bool DRAIN = false, bool ITEM = false, bool PRIO = PHASE == 3, int NIGRAM = kScreenAny,
+          bool ROWS = true>
 __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __restrict__ lds,
                                                const DevTable* __restrict__ tabs, const RunArgs& R,
                                                uint32_t& n_events, uint32_t& n_fp64, GuardBox* box = nullptr,
                                                uint32_t* pending = nullptr, LaneEl* rest = nullptr) {
   const int lane = threadIdx.x & 63;
   uint32_t k0 = (uint32_t)R.seed, k1 = (uint32_t)(R.seed >> 32);
+  const uint32_t cap = (uint32_t)(c.max_scatt < 0xFFFFFFFFll ? c.max_scatt : 0xFFFFFFFFll);
   const uint64_t n_work = PHASE == 2 ? (uint64_t)__atomic_load_n(R.park_count, __ATOMIC_RELAXED) : R.n;
 
   bool active = false, open = true;
@@ -219,7 +222,7 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
     if (!active) continue;
 
     // ---- one loop iteration of trajectory_DS / trajectory_cont_cl ----
-    if ((int64_t)step >= c.max_scatt) {  // num_scatt > maxScatt -> 'long'
+    if (step >= cap) {  // num_scatt > maxScatt -> 'long'
       const float sp[3] = {p[0] - pc[0], p[1] - pc[1], p[2] - pc[2]};  // compensated, as for other outcomes
       write_rec(&R.els[e - R.first], E.hi, d, sp, step, MCD_OUT_LONG, 0, flags);
       active = false;
@@ -306,9 +309,9 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
       const float sp[3] = {p[0] - pc[0], p[1] - pc[1], p[2] - pc[2]};
       write_rec(&R.els[e - R.first], Epre.hi, d, sp, step + 1, o1, o2, flags);
     }
-    const bool rec_row = R.rows != nullptr && e < R.row_max_electron;
+    const bool rec_row = ROWS && R.rows != nullptr && e < R.row_max_electron;
     if (!done || rec_row) f_rotate(c2, s2, u_az, d, y);  // update_direction
-    if (R.rows != nullptr) {
+    if (ROWS && R.rows != nullptr) {
       const uint64_t slot = append_slot(rec_row, R.row_cursor, R.row_cap, lane);
       if (slot != ~0ull) {
         mcd_scatter_rec* w = &R.rows[slot];
@@ -330,7 +333,8 @@ __device__ __forceinline__ void transport_loop(const DevCfg& c, const float* __r
 // allow (1 = compiler's choice, the default; others per launch).
 // PRIO: issue priority by energy, every eighth step.  NIGRAM (continuous mode):
 // the elastic screening, branched on at the launch instead of at every step.
-template <int MODE, int NCH, int MINW, int PHASE = 0, bool EXPL = false, bool PRIO = false, int NIGRAM = kScreenAny>
+template <int MODE, int NCH, int MINW, int PHASE = 0, bool EXPL = false, bool PRIO = false, int NIGRAM = kScreenAny,
+          bool ROWS = true>
 __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R) {
   extern __shared__ float lds[];
   DevTable* tabs = nullptr;
@@ -341,8 +345,8 @@ __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R
   uint32_t n_events = 0, n_fp64 = 0;
   constexpr bool drain = PHASE == 0 && MINW == 4;
   LaneEl rest;
-  transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain, false, PRIO, NIGRAM>(c, lds, tabs, R, n_events, n_fp64,
-                                                                                  nullptr, nullptr, &rest);
+  transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain, false, PRIO, NIGRAM, ROWS>(
+      c, lds, tabs, R, n_events, n_fp64, nullptr, nullptr, &rest);
   if constexpr (drain) {
     typedef typename std::conditional<MODE == MCD_MODE_DS, Fp32Ds<NCH>, Fp32Cont<EXPL>>::type P;
     // The arguments read anew: shared with the loop above, the drain's uses
@@ -372,7 +376,7 @@ static size_t svc_lds_bytes(const DevCfg& c, int block) {
            2 * sizeof(DevTable) + 15) & ~(size_t)15);
 }
 
-template <int NCH, int MINW>
+template <int NCH, int MINW, bool ROWS>
 __global__ __launch_bounds__(1024, MINW) void k_transport_svc(DevCfg c, RunArgs R) {
   extern __shared__ float lds[];
   float* pick = lds + svc_pick_offset(blockDim.x);
@@ -397,8 +401,8 @@ __global__ __launch_bounds__(1024, MINW) void k_transport_svc(DevCfg c, RunArgs 
   }
   uint32_t n_events = 0, n_fp64 = 0;
   LaneEl rest;
-  transport_loop<MCD_MODE_DS, NCH, 3, true, false, true, true>(c, pick, tabs, R, n_events, n_fp64, boxes + (w - 1),
-                                                               pending, &rest);
+  transport_loop<MCD_MODE_DS, NCH, 3, true, false, true, true, false, true, kScreenAny, ROWS>(
+      c, pick, tabs, R, n_events, n_fp64, boxes + (w - 1), pending, &rest);
   {
     // The last electrons as in k_transport_f32; their windows take the place of
     // the mailbox's slots, which are free between two posts.
@@ -975,14 +979,20 @@ static size_t with_drain(size_t used, int block, RunArgs& D) {
 // one per SIMD) 1393 and 1405, 2^19 3776 and 3307, 2^22 11186 and 10624; explicit
 // law 2^19 5764 and 5242, 2^22 27992 and 27475.  DS steps are longer and gain
 // less than it costs them (2^18 Cu 2873 and 2771, but 2^20 Au 12019 and 12217).
+// Launches without scatter rows take kernels without their tests in the step: us
+// with and without, 131072 and 2^20 electrons, Cu 2242 and 2139, 5571 and 5393, Au
+// 6058 and 5996, 11563 and 11405; explicit law 65536 1747 and 1635.
 template <int MODE, int NCH, int MINW, bool EXPL>
-static const void* f32_kernel(const DevCfg& c, int simd_waves) {
+static const void* f32_kernel(const DevCfg& c, int simd_waves, bool rows) {
+  if constexpr (MINW == 4 && MODE == MCD_MODE_DS)
+    if (!rows) return reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, false, kScreenAny, false>);
   if constexpr (MODE == MCD_MODE_CONT && MINW == 4) {
+    if (rows) return reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL>);
     if (c.elastic >= MCD_ELASTIC_NIGRAM)
-      return simd_waves >= 3 ? reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, true, 1>)
-                             : reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, false, 1>);
-    return simd_waves >= 3 ? reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, true, 0>)
-                           : reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, false, 0>);
+      return simd_waves >= 3 ? reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, true, 1, false>)
+                             : reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, false, 1, false>);
+    return simd_waves >= 3 ? reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, true, 0, false>)
+                           : reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL, false, 0, false>);
   }
   return reinterpret_cast<const void*>(&k_transport_f32<MODE, NCH, MINW, 0, EXPL>);
 }
@@ -993,7 +1003,7 @@ static hipError_t launch_f32(const DevCfg& c, const RunArgs& R, int grid, int bl
   const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
   if (R.rows || MINW != 4) D.drain = 0;
   void* args[] = {(void*)&c, (void*)&D};
-  return hipLaunchKernel(f32_kernel<MODE, NCH, MINW, EXPL>(c, R.simd_waves), dim3(grid), dim3(block), args, lds, s);
+  return hipLaunchKernel(f32_kernel<MODE, NCH, MINW, EXPL>(c, R.simd_waves, R.rows != nullptr), dim3(grid), dim3(block), args, lds, s);
 }
 
 template <int MODE, int NCH, int MINW, bool EXPL>
@@ -1001,7 +1011,7 @@ static int occ_f32(const DevCfg& c, int block, size_t used) {
   int nb = 0;
   RunArgs D;
   const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f32_kernel<MODE, NCH, MINW, EXPL>(c, 0), block, lds) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f32_kernel<MODE, NCH, MINW, EXPL>(c, 0, false), block, lds) !=
       hipSuccess)
     return 1;
   return nb < 1 ? 1 : nb;
@@ -1122,19 +1132,30 @@ hipError_t launch_transport_deferred(const DevCfg& c, const RunArgs& R, int phas
 // ---------------------------------------------------------------------------
 // Service guard (DS, FP32): one kernel, wavefront 0 of each workgroup settles
 // the guard-band picks of the others.
+// Launches without scatter rows take a kernel without their tests in the step
+// (us with and without, 2^22 electrons: Cu, 7 channels 14451 and 14166, Al 6780
+// and 6633, Si 12988 and 12636).  From 9 channels on it spills more at 64 VGPRs
+// (Au, 11 channels 29703 and 33185), and the one with the tests serves both.
+template <int NCH>
+constexpr bool kLean = NCH <= 8;
+
 template <int NCH, int MINW>
 static hipError_t svc_nch(const DevCfg& c, const RunArgs* R, int grid, int block, size_t lds, hipStream_t s,
                           int* occ) {
   if (occ) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_transport_svc<NCH, MINW>, block, lds) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_transport_svc<NCH, MINW, !kLean<NCH>>, block, lds) !=
+        hipSuccess)
       nb = 1;
     *occ = nb < 1 ? 1 : nb;
     return hipSuccess;
   }
   RunArgs D = *R;
   D.drain = R->rows ? 0 : kDrain;
-  hipLaunchKernelGGL((k_transport_svc<NCH, MINW>), dim3(grid), dim3(block), lds, s, c, D);
+  if (R->rows || !kLean<NCH>)
+    hipLaunchKernelGGL((k_transport_svc<NCH, MINW, true>), dim3(grid), dim3(block), lds, s, c, D);
+  else
+    hipLaunchKernelGGL((k_transport_svc<NCH, MINW, !kLean<NCH>>), dim3(grid), dim3(block), lds, s, c, D);
   return hipGetLastError();
 }
 

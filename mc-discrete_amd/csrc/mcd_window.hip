@@ -59,10 +59,10 @@ static size_t window_lds_bytes(const DevCfg& c) {
 //   DS FP64, 1.5 and 4 (Cu; 4000: 1967 at 32, 1709 at 16; 8192: 2623 at 16,
 //     2482 at 8; 16000: 3812 at 8, 4116 at 4; 65000: 9846 at 4, 10656 at 1;
 //     131072: 16980 at 4, 16270 at 1)
-//   continuous, 1 and 3.25 (Au 30 keV JL 70 deg; 2000: 424 at 32; 10007: 646 at 4;
-//     32768: 833 at 4, 1380 at 1; 40000: 1109, 1386; 50021: 1374, 1391; 60000: 1412,
-//     1396), with the explicit law 1 and 1 (16384: 1176 at 4, 1642 at 1; 32768:
-//     1747, 1760; 40000: 2347, 1761)
+//   continuous, 1 and 3 (Au 30 keV JL 70 deg; 2000: 424 at 32; 10007: 646 at 4;
+//     32768: 833 at 4, 1380 at 1; 40000: 1093, 1340; 50021: 1320 to 1390, 1315;
+//     60000: 1412, 1320), with the explicit law 1 and 1 (16384: 1176 at 4, 1642 at
+//     1; 32768: 1747, 1600; 40000: 2347, 1600)
 // Pick tables beyond 64 KB of LDS with the staged steps (512 nodes: 27 KB with
 // 7 channels) take the other kernels, as does continuous mode in FP64.
 int window_log2_lanes(const DevCfg& c, int precision, uint64_t n, int n_cu) {
@@ -70,7 +70,7 @@ int window_log2_lanes(const DevCfg& c, int precision, uint64_t n, int n_cu) {
   if (ds && !f64 && window_lds_bytes<Fp32Ds<4>, false>(c) > 64 * 1024) return 0;
   if (!ds && f64) return 0;
   const double wide = ds ? (f64 ? 1.5 : 3.75) : 1.;
-  const double quad = ds ? (f64 ? 4. : 5.) : (c.bethe == MCD_BETHE_EXPLICIT ? 1. : 3.25);
+  const double quad = ds ? (f64 ? 4. : 5.) : (c.bethe == MCD_BETHE_EXPLICIT ? 1. : 3.);
   const double lanes = (double)n_cu * 4 * 64;  // one wavefront per SIMD
   for (int lg = 6; lg > 2; --lg)
     if ((double)n * (1 << lg) <= wide * lanes) return lg;

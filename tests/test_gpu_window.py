@@ -166,9 +166,21 @@ def test_continuous_priority_form_equals_the_others(law, n):
     _same(tr.run(n, seed=3, first=9), tr.run(n, seed=3, first=9, waves_per_simd=5))
 
 
-# quads to 3.25 wavefronts per SIMD (53248 electrons on 256 CUs), a kernel per screening on either side
+# quads to 3 wavefronts per SIMD (49152 electrons on 256 CUs), a kernel per screening on either side
 @pytest.mark.parametrize("elastic", ["Ruth_vanilla", "Ruth_nigram"])
-@pytest.mark.parametrize("law,n", [("JL", 53248), ("classical", 53249), ("JL", 196608), ("explicit", 16385)])
+@pytest.mark.parametrize("law,n", [("JL", 49152), ("classical", 49153), ("JL", 196608), ("explicit", 16385)])
 def test_continuous_screenings_equal_the_general_form(elastic, law, n):
     tr = engine.Transport("Au", 6000.0, 1000.0, s_tilt=60.0, mode="cont", bethe_model=law, elastic=elastic)
     _same(tr.run(n, seed=5, first=2), tr.run(n, seed=5, first=2, waves_per_simd=5))
+
+
+# kernels with and without the tests for scatter rows, past the sizes of several lanes per electron
+@pytest.mark.parametrize("kw,n", [(dict(), 81921), (dict(material="Au", E0=5000.0), 81921),
+                                  (dict(material="Al", E0=5000.0, max_scatt=40), 90000)], ids=str)
+def test_rows_do_not_change_the_records(kw, n):
+    tr = _transport(**kw)
+    for guard in ("inline", "service"):
+        a = tr.run(n, seed=2, guard=guard)
+        b = tr.run(n, seed=2, guard=guard, scats=True, scat_max_electron=50)
+        assert a.els.tobytes() == b.els.tobytes()
+        assert len(b.scats) == a.els["n_scatt"][:50].sum()
