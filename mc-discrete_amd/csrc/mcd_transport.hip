@@ -507,7 +507,9 @@ __device__ __forceinline__ void run_item(const DevCfg& c, const DevTable* tabs, 
   // the table descriptors from the LDS copy: the per-lane Moller / Gryzinski select reads LDS
   R.drain = DRAIN ? kDrain : 0;
   LaneEl rest;
-  transport_loop<MODE, NCH, MODE == MCD_MODE_DS ? PHASE : 0, PERIOD, EXPL, false, DRAIN, true>(
+  constexpr int kPhase = MODE == MCD_MODE_DS ? PHASE : 0;
+  // items store no scatter rows
+  transport_loop<MODE, NCH, kPhase, PERIOD, EXPL, false, DRAIN, true, kPhase == 3, kScreenAny, false>(
       c, pick, tabs, R, ne, nf, box, pending, &rest);
   if constexpr (DRAIN) {
     typedef typename std::conditional<MODE == MCD_MODE_DS, Fp32DsItem<NCH>, Fp32Cont<EXPL>>::type P;
