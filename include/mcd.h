@@ -243,8 +243,9 @@ typedef struct mcd_launch {
  * block may then be 128 to 1024).  Records are identical in every form.
  * Without a flag (and without block or waves_per_simd), mcd_forward runs DS
  * launches of at least 2^21 electrons served and smaller ones inline; those too
- * small to fill the GPU with one lane per electron (up to 384 electrons per
- * CU) run with 4 to 64 lanes per electron, guard inline;
+ * small to fill the GPU with one lane per electron (up to 320 electrons per CU;
+ * FP64 256, continuous mode 192, explicit law 64) run with 4 to 64 lanes per
+ * electron, guard inline;
  * mcd_batch_run runs inline unless another form is asked for (the faster form
  * depends on the configuration; mcd/autotune.py measures it).  Setting more
  * than one flag is an error. */
