@@ -162,6 +162,14 @@ constexpr float kXCut = 30.f;                   // exp(-30) ~ 1e-13: no exit con
 constexpr float kWMin = 1e-12f;                 // weight below which a replay ends
 constexpr uint32_t kBwdStepCap = 1u << 22;
 
+// Sums (value and slot derivatives): FP32 in a lane over its electrons, then over
+// the lanes of a wavefront; FP64 over wavefronts.  A launch with one electron per
+// lane places its electrons by position, so it repeats to FP64 rounding.  A
+// larger one hands electrons out as lanes become free, so two of its runs differ
+// by the FP32 rounding of other lane sums (2^20 electrons of Cu 20 keV: 9e-9 to
+// 7e-7 of the gradient's norm).  FP64 sums over electrons repeat to 1e-14, but
+// lie 1e-7 to 7e-7 from the FP32 ones, three times as far as those from each
+// other: they would change every large gradient.
 // LDS: the node table, the histogram or the upstream gradients, the two
 // loss-table descriptors.  Bound by vector issue while a large launch fills the
 // chip (0.83 of the ceiling) and by the latency of a step (3 us on a lone
@@ -210,6 +218,12 @@ __global__ __launch_bounds__(256) void k_backward(DevCfg c, BwdArgs A) {
 
   bool active = false, open = true;
   WaveQueue wq;
+  // one electron per lane: the wavefront's only reservation is its own 64
+  const bool one_each = A.n <= (uint64_t)gridDim.x * blockDim.x;
+  if (one_each) {
+    wq.next = (uint64_t)blockIdx.x * blockDim.x + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
+    wq.end = wq.next + 64;
+  }
   uint64_t e = 0;
   uint32_t step = 0;
   float E = 0.f, z = 0.f, w = 0.f;
@@ -226,6 +240,7 @@ __global__ __launch_bounds__(256) void k_backward(DevCfg c, BwdArgs A) {
       const uint64_t idle = __ballot(!active);
       if (idle) {
         const uint64_t idx = refill_index(wq, A.queue, idle, lane, A.n, open);
+        if (one_each) open = false;
         if (!active) {
           if (idx < A.n) {
             active = true;
