@@ -616,7 +616,9 @@ __device__ __forceinline__ void window_loop(const DevCfg& c, const RunArgs& R, c
     const bool rec_row = ROWS && active && s.e < R.row_max_electron;
     const Real thick = P::thickness(c);
     int ran = 0;  // steps executed
-    Real tz = 1;  // depth after the last executed step (an exit ends the window)
+    // depth after the last executed step (an exit ends the window); NaN, neither
+    // in front nor behind, for a window that passes whole inside the film
+    Real tz = (Real)__builtin_nan("");
     bool go = active && m > 0;
     Real rx = 0, ry = 0, rz = 0, rdx = 0, rdy = 0, rdz = 0;  // ROWS: lane j's step
     // selects instead of branches: no lane leaves the loop before the last
