@@ -9,7 +9,9 @@ second kernel whose first phase carries no FP64 code, or served by wavefront 0
 of each workgroup through LDS (one kernel whose transport code carries no
 FP64), and ``refill_period``, the compaction period: a wavefront refills its
 idle lanes with new electrons every that many steps (fewer refill passes,
-lanes idle a little longer).  Records are identical for every shape.
+lanes idle a little longer).  The library's own shape is a candidate too (the
+only one with several lanes per electron in small launches).  Records are
+identical for every shape.
 
 Batched runs (``tune_batch``):
 
@@ -19,7 +21,7 @@ The batched kernel has four shape choices that trade against each other:
   the wavefront's LDS slice.  More nodes give a narrower FP64 guard band and a
   finer mean-free-path interpolation but a larger slice, so fewer workgroups
   fit a CU; 0 sizes each table to the default 8 KB slice.
-* ``block`` — threads per workgroup (64, 128 or 256).
+* ``block`` — threads per workgroup (64, 128 or 256; 0: the library's choice).
 * ``guard`` — where DS items take the FP64 guard pick: ``"deferred"`` (a
   first phase without FP64 code parks those electrons, a second resumes them),
   ``"inline"`` (one phase, more registers, fewer resident wavefronts) or
@@ -42,7 +44,11 @@ import json
 import os
 import time
 
+# block 0: the library's own choice (workgroups of one wavefront where LDS then
+# holds more of them, a drain of the last electrons in short runs)
 CANDIDATES = (
+    dict(block=0, pick_nodes=0, guard="inline"),
+    dict(block=0, pick_nodes=128, guard="inline"),
     dict(block=1024, pick_nodes=128, guard="service"),
     dict(block=128, pick_nodes=128, guard="inline"),
     dict(block=256, pick_nodes=128, guard="inline"),
@@ -61,7 +67,9 @@ def _name(c):
             f"refill_period={c.get('refill_period', 1)}")
 
 
+# the first: the library's own shape, several lanes per electron in small launches
 TRANSPORT_CANDIDATES = (
+    dict(block=0, waves_per_simd=0, guard=None, refill_period=1),
     dict(block=256, waves_per_simd=4, guard="inline", refill_period=1),
     dict(block=128, waves_per_simd=4, guard="inline", refill_period=1),
     dict(block=256, waves_per_simd=5, guard="inline", refill_period=1),
@@ -146,7 +154,7 @@ def tune_transport(tr, n=1 << 22, seed=1, candidates=TRANSPORT_CANDIDATES, reps=
     key = transport_key(tr, n) + hashlib.sha1(",".join(_tname(c) for c in candidates).encode()).hexdigest()[:8]
     from . import _abi
     if tr.mode != _abi.MODE_DS:  # continuous mode has no guard pick to place
-        candidates = tuple(c for c in candidates if c["guard"] == "inline")
+        candidates = tuple(c for c in candidates if c["guard"] in (None, "inline"))
     if use_cache:
         hit = _load(path).get(key)
         if hit and any(_tname(hit) == _tname(c) for c in candidates):

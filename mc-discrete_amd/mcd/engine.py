@@ -116,7 +116,7 @@ class Transport:
         self.tol_E, self.tol_W = tol_E, tol_W
         self.grids = grids
         # launch shape used when a launch leaves block / waves_per_simd / guard
-        # at their defaults; set by tune()
+        # at their defaults; set by tune(), with the electrons n it was timed on
         self.tuned = None
         self._tables = C.c_void_p()
         ctx = context(device)
@@ -237,7 +237,7 @@ class Transport:
         or "service" -- where the DS FP64 guard pick runs (same records in
         every form).  refill_period: the compaction period, idle lanes take
         new electrons every refill_period steps (0: every step)."""
-        if self.tuned is not None and precision == _abi.PREC_FP32:
+        if self.tuned is not None and precision == _abi.PREC_FP32 and self._tuned_covers(n):
             block = block or self.tuned["block"]
             waves_per_simd = waves_per_simd or self.tuned["waves_per_simd"]
             guard = guard or self.tuned["guard"]
@@ -254,14 +254,30 @@ class Transport:
                                 els.data_ptr(), C.byref(sb) if sb is not None else None, counters.data_ptr(),
                                 C.byref(la), s), ctx)
 
+    def _several_lanes(self, n):
+        """Whether the library's own shape takes several lanes per electron for
+        n electrons (FP32; sizes per CU as in mcd.h, mcd_launch)."""
+        per_cu = 320 if self.mode == _abi.MODE_DS else (64 if self.cfg.bethe_model == _abi.BETHE_EXPLICIT else 192)
+        return n <= per_cu * torch.cuda.get_device_properties(self.device).multi_processor_count
+
+    def _tuned_covers(self, n):
+        """Whether the tuned shape is used for n electrons: a shape timed on a
+        large launch is not used for one that takes several lanes per electron
+        without it (10007 electrons of Cu 20 keV: 0.61 ms, and 1.97 to 3.83 ms at
+        the other candidates)."""
+        at = self.tuned.get("n")
+        return at is None or self._several_lanes(at) or not self._several_lanes(n)
+
     def tune(self, n=1 << 22, **kw):
         """Time the launch shapes of mcd.autotune.TRANSPORT_CANDIDATES on n
         electrons of this configuration, keep the fastest for later launches
-        (records are the same for every shape) and return the tuner's report."""
+        (records are the same for every shape) and return the tuner's report.
+        A shape of large launches is not used for small ones (several lanes
+        per electron at the library's own shape)."""
         from .autotune import tune_transport
         res = tune_transport(self, n, **kw)
         self.tuned = dict(block=res["block"], waves_per_simd=res["waves_per_simd"], guard=res["guard"],
-                          refill_period=res.get("refill_period", 1))
+                          refill_period=res.get("refill_period", 1), n=int(n))
         return res
 
     def run(self, n, seed=1, first=0, config_id=0, scats=False, scat_max_electron=None, scat_capacity=None,
