@@ -1113,6 +1113,7 @@ struct mcd_batch {
   hipStream_t graph_stream;
   int graph_block, graph_grid, graph_deferred;  // graph_deferred: the guard form the graph was captured with
   uint32_t graph_refill;                        // the compaction period less one it was captured with
+  bool graph_drain;                             // whether it was captured with a drain
 };
 
 static double work_per_electron(const mcd_config& c) {
@@ -1359,7 +1360,7 @@ extern "C" int mcd_batch_run(mcd_ctx* ctx, mcd_batch* b, uint64_t seed, uint64_t
     return MCD_OK;
   }
   if (!b->graph || b->graph_seed != seed || b->graph_counters != counters || b->graph_block != block ||
-      b->graph_deferred != form || b->graph_refill != refill) {
+      b->graph_deferred != form || b->graph_refill != refill || b->graph_drain != drain) {
     if (b->graph) { (void)hipGraphExecDestroy(b->graph); b->graph = nullptr; }
     if (!b->capture_stream) HIP_TRY(ctx, hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
     HIP_TRY(ctx, hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal));
@@ -1376,6 +1377,7 @@ extern "C" int mcd_batch_run(mcd_ctx* ctx, mcd_batch* b, uint64_t seed, uint64_t
     b->graph_block = block;
     b->graph_deferred = form;
     b->graph_refill = refill;
+    b->graph_drain = drain;
   }
   HIP_TRY(ctx, hipGraphLaunch(b->graph, s));
   return MCD_OK;
