@@ -213,7 +213,7 @@ enum {
   MCD_CNT_LONG = 5,
   MCD_CNT_FP64_PICKS = 6, /* picks settled by the FP64 guard */
   MCD_CNT_SCAT_ROWS = 7,  /* scatter rows requested (may exceed capacity) */
-  MCD_CNT_QUEUE = 8,      /* internal: the launch's work counter (mcd_forward resets it) */
+  MCD_CNT_QUEUE = 8,      /* internal: the launch's work counter (mcd_forward resets it where it uses one) */
   MCD_CNT_GUARD_TIMEOUTS = 9, /* guard picks left unsettled: a served-guard wait that timed out, or
                                  a parked electron the resume kernel could not place (must be 0;
                                  otherwise the launch's records are not valid) */

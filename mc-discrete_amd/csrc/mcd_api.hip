@@ -1013,7 +1013,6 @@ static int forward_impl(mcd_ctx* ctx, const mcd_config* cfg, const mcd_tables* t
   // several lanes per electron, unless a placement or a shape is asked for
   const int wlg = !guard_flags && !shape_given ? window_log2_lanes(c, precision, n, ctx->n_cu) : 0;
   if (wlg) {
-    HIP_TRY(ctx, launch_fill_u64(q, 0ull, 1, s));
     HIP_TRY(ctx, launch_window(c, R, precision, wlg, s));
   } else if (service) {
     // wavefront 0 of each workgroup serves the guard; the others carry electrons

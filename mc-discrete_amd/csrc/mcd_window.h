@@ -149,6 +149,7 @@ __device__ __forceinline__ void ds_energies(const DevCfg& c, const float* __rest
 // FP32, energies as float pairs.  A staged step: path, cos and sin of the polar
 // angle, cos and |sin| of the azimuth.
 struct Fp32Base {
+  static constexpr int kWaves = 2;  // wavefronts per SIMD of k_window, at least
   typedef float Real;
   typedef F2 Energy;
   struct alignas(8) Staged {
@@ -374,6 +375,9 @@ struct Fp32Cont : Fp32Base {
 #pragma clang fp contract(off)
 template <int NCH>
 struct Fp64Ds {
+  // 65000 electrons, us at 2 and 3: Cu, 7 channels 11020 and 9860, Si, 6 channels
+  // 4770 and 4560; Au with 11 channels 12500 and, with spills, 12870
+  static constexpr int kWaves = NCH <= 7 ? 3 : 2;
   typedef double Real;
   typedef double Energy;
   static constexpr bool kServed = false;
@@ -485,6 +489,20 @@ struct WinEl {
   uint32_t ctr1, step, flags;
 };
 
+// The start of electron e, component comp of each vector.
+template <class P>
+__device__ __forceinline__ WinEl<P> win_start(const DevCfg& c, uint64_t e, int comp) {
+  WinEl<P> s;
+  s.p = s.pc = 0;
+  s.d = P::dir0(c, comp);
+  s.y = comp == 1 ? 1 : 0;
+  s.E = P::start(c);
+  s.e = e;
+  s.ctr1 = c.config_id | (uint32_t)(e >> 32) << 16;
+  s.step = s.flags = 0;
+  return s;
+}
+
 // A window is G steps; in continuous mode at least 16, up to 4 (kTurns) a lane:
 // its chain gains nothing from the lanes, and the work of a window beside its
 // steps (1100 cycles) is spread over more of them.
@@ -502,11 +520,9 @@ __host__ __device__ inline size_t win_stage_offset(const DevCfg& c) {
   return ((size_t)tab_offset_floats(nf) * sizeof(float) + 2 * sizeof(DevTable) + 15) & ~(size_t)15;
 }
 
-// The loop of one wavefront over its electrons, 2^lg lanes each (lg grows as
-// fewer are left).  REFILL: a launch of its own, whose first electrons are
-// those by position and whose later ones come from the work counter; otherwise
-// the electrons in s (active lanes) are run to their end.
-template <class P, bool ROWS, int M, bool REFILL>
+// A wavefront's electrons (those of the active lanes, 2^lg lanes each) to their
+// end; lg grows as fewer are left.
+template <class P, bool ROWS, int M>
 __device__ __forceinline__ void window_loop(const DevCfg& c, const RunArgs& R, const float* __restrict__ lds,
                                             const DevTable* __restrict__ tabs, typename P::Staged* win, int lg,
                                             WinEl<P> s, bool active, uint32_t& n_events, uint32_t& n_fp64) {
@@ -514,43 +530,14 @@ __device__ __forceinline__ void window_loop(const DevCfg& c, const RunArgs& R, c
   const int lane = threadIdx.x & 63;
   uint32_t k0 = (uint32_t)R.seed, k1 = (uint32_t)(R.seed >> 32);
   const int comp = (lane & 3) == 3 ? 0 : (lane & 3);
-  const Real dir0 = P::dir0(c, comp);
-  const uint64_t slots = REFILL ? (uint64_t)gridDim.x * (blockDim.x >> lg) : 0;
-  uint64_t next = REFILL ? (((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> lg) : 0;
-  bool first = true, open = REFILL;
 
   while (true) {
     // the key words stay loop-carried SGPR values (see transport_loop)
     asm volatile("" : "+s"(k0), "+s"(k1));
     Group g(lg, lane);
-    if (REFILL && open) {
-      const uint64_t idle = __ballot(!active && g.j == 0);
-      if (idle) {
-        if (!first) {
-          const int leader = __ffsll((unsigned long long)idle) - 1;
-          unsigned long long b = 0;
-          if (lane == leader) b = atomicAdd(R.queue, (unsigned long long)__popcll(idle));
-          next = slots + lane_u64(b, leader) + __popcll(idle & ((1ull << g.base) - 1ull));
-        }
-        first = false;
-        if (!active && next < R.n) {
-          active = true;
-          s.e = R.first + next;
-          s.ctr1 = c.config_id | (uint32_t)(s.e >> 32) << 16;
-          s.step = 0;
-          s.flags = 0;
-          s.E = P::start(c);
-          s.p = s.pc = 0;
-          s.d = dir0;
-          s.y = comp == 1 ? 1 : 0;
-        }
-        // an index past the end: every later one is past it too
-        open = slots < R.n && !__any(!active);
-      }
-    }
     const uint64_t live = __ballot(active && g.j == 0);
     if (!live) break;
-    if ((!REFILL || !open) && lg < 6 && 2 * __popcll(live) * g.G <= 64) {
+    if (lg < 6 && 2 * __popcll(live) * g.G <= 64) {
       // fewer electrons than half the groups: wider groups, longer windows
       const int n = __popcll(live);
       while (lg < 6 && (n << (lg + 1)) <= 64) ++lg;
@@ -782,7 +769,7 @@ __device__ __forceinline__ void window_drain(const DevCfg& c, const RunArgs& R, 
   s.ctr1 = c.config_id | (uint32_t)(s.e >> 32) << 16;
   s.step = shfl_any(q.step, src);
   s.flags = shfl_any(q.flags, src);
-  window_loop<P, false, 1, false>(c, R, lds, tabs, win, lg, s, mine < n, n_events, n_fp64);
+  window_loop<P, false, 1>(c, R, lds, tabs, win, lg, s, mine < n, n_events, n_fp64);
 }
 
 }  // namespace mcd

@@ -10,7 +10,7 @@
 namespace mcd {
 
 template <class P, bool ROWS>
-__global__ __launch_bounds__(256, 2) void k_window(DevCfg c, RunArgs R, int lg) {
+__global__ __launch_bounds__(256, ROWS ? 2 : P::kWaves) void k_window(DevCfg c, RunArgs R, int lg) {
   constexpr int M = win_turns<P, ROWS>();
   extern __shared__ float lds[];
   const DevTable* tabs = nullptr;
@@ -30,7 +30,10 @@ __global__ __launch_bounds__(256, 2) void k_window(DevCfg c, RunArgs R, int lg) 
       reinterpret_cast<typename P::Staged*>(reinterpret_cast<char*>(lds) + win_stage_offset<P>(c)) + win_stage(M) * wib;
   __syncthreads();
   uint32_t n_events = 0, n_fp64 = 0;
-  window_loop<P, ROWS, M, true>(c, R, lds, tabs, win, lg, WinEl<P>{}, false, n_events, n_fp64);
+  // one group of lanes for each electron of the launch
+  const uint64_t idx = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> lg;
+  const int comp = (lane & 3) == 3 ? 0 : (lane & 3);
+  window_loop<P, ROWS, M>(c, R, lds, tabs, win, lg, win_start<P>(c, R.first + idx, comp), idx < R.n, n_events, n_fp64);
   const uint64_t cnt[2] = {n_events, n_fp64};
   wave_add_counters(R.counters + MCD_CNT_EVENTS, cnt, 1, lane);
   wave_add_counters(R.counters + MCD_CNT_FP64_PICKS, cnt + 1, 1, lane);
