@@ -343,7 +343,7 @@ __global__ __launch_bounds__(256, MINW) void k_transport_f32(DevCfg c, RunArgs R
     __syncthreads();
   }
   uint32_t n_events = 0, n_fp64 = 0;
-  constexpr bool drain = PHASE == 0 && MINW == 4;
+  constexpr bool drain = PHASE == 0 && MINW == 4 && !ROWS;
   LaneEl rest;
   transport_loop<MODE, NCH, PHASE, true, EXPL, false, drain, false, PRIO, NIGRAM, ROWS>(
       c, lds, tabs, R, n_events, n_fp64, nullptr, nullptr, &rest);
@@ -376,6 +376,13 @@ static size_t svc_lds_bytes(const DevCfg& c, int block) {
            2 * sizeof(DevTable) + 15) & ~(size_t)15);
 }
 
+// Launches without scatter rows take a kernel without their tests in the step
+// (us with and without, 2^22 electrons: Cu, 7 channels 14451 and 14166, Al 6780
+// and 6633, Si 12988 and 12636).  From 9 channels on it spills more at 64 VGPRs
+// (Au, 11 channels 29703 and 33185), and the one with the tests serves both.
+template <int NCH>
+constexpr bool kLean = NCH <= 8;
+
 template <int NCH, int MINW, bool ROWS>
 __global__ __launch_bounds__(1024, MINW) void k_transport_svc(DevCfg c, RunArgs R) {
   extern __shared__ float lds[];
@@ -400,10 +407,11 @@ __global__ __launch_bounds__(1024, MINW) void k_transport_svc(DevCfg c, RunArgs 
     return;
   }
   uint32_t n_events = 0, n_fp64 = 0;
+  constexpr bool drain = !ROWS || !kLean<NCH>;  // launches with rows have none
   LaneEl rest;
-  transport_loop<MCD_MODE_DS, NCH, 3, true, false, true, true, false, true, kScreenAny, ROWS>(
+  transport_loop<MCD_MODE_DS, NCH, 3, true, false, true, drain, false, true, kScreenAny, ROWS>(
       c, pick, tabs, R, n_events, n_fp64, boxes + (w - 1), pending, &rest);
-  {
+  if constexpr (drain) {
     // The last electrons as in k_transport_f32; their windows take the place of
     // the mailbox's slots, which are free between two posts.
     typedef Fp32DsServed<NCH> P;
@@ -1002,8 +1010,7 @@ static const void* f32_kernel(const DevCfg& c, int simd_waves, bool rows) {
 template <int MODE, int NCH, int MINW, bool EXPL>
 static hipError_t launch_f32(const DevCfg& c, const RunArgs& R, int grid, int block, size_t used, hipStream_t s) {
   RunArgs D = R;
-  const size_t lds = MINW == 4 ? with_drain(used, block, D) : used;
-  if (R.rows || MINW != 4) D.drain = 0;
+  const size_t lds = MINW == 4 && !R.rows ? with_drain(used, block, D) : used;
   void* args[] = {(void*)&c, (void*)&D};
   return hipLaunchKernel(f32_kernel<MODE, NCH, MINW, EXPL>(c, R.simd_waves, R.rows != nullptr), dim3(grid), dim3(block), args, lds, s);
 }
@@ -1134,13 +1141,6 @@ hipError_t launch_transport_deferred(const DevCfg& c, const RunArgs& R, int phas
 // ---------------------------------------------------------------------------
 // Service guard (DS, FP32): one kernel, wavefront 0 of each workgroup settles
 // the guard-band picks of the others.
-// Launches without scatter rows take a kernel without their tests in the step
-// (us with and without, 2^22 electrons: Cu, 7 channels 14451 and 14166, Al 6780
-// and 6633, Si 12988 and 12636).  From 9 channels on it spills more at 64 VGPRs
-// (Au, 11 channels 29703 and 33185), and the one with the tests serves both.
-template <int NCH>
-constexpr bool kLean = NCH <= 8;
-
 template <int NCH, int MINW>
 static hipError_t svc_nch(const DevCfg& c, const RunArgs* R, int grid, int block, size_t lds, hipStream_t s,
                           int* occ) {
