@@ -1011,7 +1011,8 @@ static int forward_impl(mcd_ctx* ctx, const mcd_config* cfg, const mcd_tables* t
   const uint64_t want = (n + block - 1) / block;
   // launches too small to fill the chip with one lane per electron take
   // several lanes per electron, unless a placement or a shape is asked for
-  const int wlg = !guard_flags && !shape_given ? window_log2_lanes(c, precision, n, ctx->n_cu) : 0;
+  // (MCD_MINW is one)
+  const int wlg = !guard_flags && !shape_given && !getenv("MCD_MINW") ? window_log2_lanes(c, precision, n, ctx->n_cu) : 0;
   if (wlg) {
     HIP_TRY(ctx, launch_window(c, R, precision, wlg, s));
   } else if (service) {

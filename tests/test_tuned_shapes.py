@@ -67,3 +67,32 @@ def test_tuning_a_small_launch_can_keep_several_lanes_per_electron(kw):
     assert (tr.tuned["block"], tr.tuned["guard"], tr.tuned["n"]) == (0, None, 10007), res["ms"]
     assert tr.run(10007, seed=2).els.tobytes() == ref.els.tobytes()
     assert tr.run(100001, seed=2).els.tobytes() == tr.run(100001, seed=2, waves_per_simd=5).els.tobytes()
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="no GPU")
+def test_an_asked_for_register_budget_is_a_shape(monkeypatch):
+    """MCD_MINW sets the wavefronts per SIMD of small launches too: one lane per
+    electron, over three times as long for 10007 electrons."""
+    import torch
+    tr = engine.Transport("Cu", 20000.0, 1000.0, s_tilt=70.0, Wc=50.0, tol_E=1e-2, tol_W=1e-2)
+    n = 10007
+    els = torch.empty(n * _abi.ELECTRON_DTYPE.itemsize, dtype=torch.uint8, device="cuda")
+    cnt = torch.zeros(_abi.NCOUNTERS, dtype=torch.int64, device="cuda")
+
+    def best():
+        t = []
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            tr.launch(n, els, cnt)
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b))
+        return min(t), els.cpu().numpy().tobytes()
+
+    own, rec = best()
+    monkeypatch.setenv("MCD_MINW", "5")
+    asked, same = best()
+    equal = same == rec
+    assert equal and asked > 2 * own, (asked, own)
