@@ -326,8 +326,7 @@ static int build_pick_tables(mcd_ctx* ctx, mcd_tables* const* ts, const int* n_n
     t->lnE0 = log(cfg.Emin);
     t->dln = (log(cfg.E0) - t->lnE0) / (double)(t->n_nodes - 1);
     t->delta = 0.f;
-    const size_t nf = (size_t)t->n_nodes * t->stride;
-    if (hipMalloc(&t->nodes, nf * sizeof(float) + sizeof(PickSummary)) != hipSuccess)
+    if (hipMalloc(&t->nodes, pick_bytes(t->n_nodes, t->stride)) != hipSuccess)
       return set_err(ctx, MCD_ERR_NOMEM, "hipMalloc for the pick table failed");
     const DevCfg c = make_devcfg(cfg, t, 0);
     HIP_TRY(ctx, launch_pick_nodes(c, t->n_nodes, t->lnE0, t->dln, t->nodes, t->stride, 0));

@@ -154,11 +154,15 @@ hipError_t launch_pick_nodes(const DevCfg& c, int n_nodes, double lnE0, double d
                              hipStream_t s);
 hipError_t launch_pick_check(const DevCfg& c, float* nodes, hipStream_t s);
 constexpr int kPickChecks = 16;  // check points per cell
-// Kept behind the last node of a pick table while it is built.
+// Kept behind the last node of a pick table while it is built, with a byte for
+// each cell after it (whether it is exact).
 struct PickSummary {
   uint32_t max_err;  // bits of the largest interpolation error (not negative)
   int n_swap, n_exact;
 };
+inline size_t pick_bytes(int n_nodes, int stride) {
+  return (size_t)n_nodes * stride * sizeof(float) + sizeof(PickSummary) + (size_t)n_nodes;
+}
 hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, int n, hipStream_t s);
 hipError_t launch_unmask(const float* src, float* dst, size_t n, hipStream_t s);
 hipError_t launch_mask(const float* src, float* dst, size_t n, hipStream_t s);

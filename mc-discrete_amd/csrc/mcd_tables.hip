@@ -1,11 +1,11 @@
 // mcd_tables.hip — device-side table construction.
 //
 // * k_build_cdf: the inverse-CDF energy-loss rows of probTable.computeBlock
-//   (MC/tools/probTables.py:415-462).  One thread per energy row; FP64
+//   (MC/tools/probTables.py:415-462).  One wavefront per energy row; FP64
 //   trapezoids and cumulative sums (rounded to float32 once), or the float32
 //   arithmetic of the reference.  The mask W[j+1] > (E - E_F)/2 is evaluated in
 //   float32 exactly as the reference's float32 arrays do (:429-439).
-// * k_pick_nodes / k_pick_cells / k_pick_check: the LDS pick table (sorted
+// * k_pick_nodes / k_pick_cells / k_pick_check / k_pick_exact: the LDS pick table (sorted
 //   cumulative channel probabilities and ln mfp on a ln E grid), the kinds of its
 //   cells, and its interpolation-error check against the exact FP64 pick, which
 //   sets the guard band.  What the host needs of them is a PickSummary.
@@ -434,9 +434,16 @@ __device__ __forceinline__ void pick_point(const DevCfg& c, int k, int m, float&
   bad = mism != 0;
 }
 
+// The cells' verdicts, behind the summary.
+__device__ __forceinline__ uint8_t* pick_verdicts(float* nodes, int n_nodes, int stride) {
+  return reinterpret_cast<uint8_t*>(nodes + (size_t)n_nodes * stride) + sizeof(PickSummary);
+}
+
 // 16 lanes to a cell.  A cell with a bad point, or an error that is NaN or above
 // 1e-4 (badly resolved), becomes exact; the largest error of the others is the
-// table's.
+// table's.  In cells a few ulp of ln E wide a point can fall into a neighbour
+// (8192 nodes from 1000 to 1100 eV: 1 % of them), so the cells stay as they are
+// until every point is checked (k_pick_exact).
 template <int NCH>
 __global__ __launch_bounds__(64) void k_pick_check(DevCfg c, float* nodes) {
   static_assert(kPickChecks == 16, "16 lanes share a cell");
@@ -453,14 +460,18 @@ __global__ __launch_bounds__(64) void k_pick_check(DevCfg c, float* nodes) {
   const uint64_t any_bad = (__ballot(bad) >> ((threadIdx.x & 63) & ~(kPickChecks - 1))) & 0xFFFFull;
   if (m) return;
   PickSummary* sum = reinterpret_cast<PickSummary*>(nodes + (size_t)c.pick.n_nodes * c.pick.stride);
-  float* meta = nodes + (size_t)k * c.pick.stride + NCH + 1;
-  const uint32_t hi = __float_as_uint(*meta);
-  if ((hi & kMetaExact) || any_bad || (double)ek > 1e-4) {
-    *meta = __uint_as_float(hi | kMetaExact);
-    atomicAdd(&sum->n_exact, 1);
-  } else {
-    atomicMax(&sum->max_err, __float_as_uint(ek));
-  }
+  const uint32_t hi = __float_as_uint(nodes[(size_t)k * c.pick.stride + NCH + 1]);
+  const bool exact = (hi & kMetaExact) || any_bad || (double)ek > 1e-4;
+  pick_verdicts(nodes, c.pick.n_nodes, c.pick.stride)[k] = exact;
+  if (exact) atomicAdd(&sum->n_exact, 1);
+  else atomicMax(&sum->max_err, __float_as_uint(ek));
+}
+
+__global__ void k_pick_exact(int n_nodes, int n_ch, float* nodes, int stride) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k + 1 >= n_nodes || !pick_verdicts(nodes, n_nodes, stride)[k]) return;
+  float* meta = nodes + (size_t)k * stride + n_ch + 1;
+  *meta = __uint_as_float(__float_as_uint(*meta) | kMetaExact);
 }
 
 hipError_t launch_pick_check(const DevCfg& c, float* nodes, hipStream_t s) {
@@ -476,6 +487,8 @@ hipError_t launch_pick_check(const DevCfg& c, float* nodes, hipStream_t s) {
     case 11: hipLaunchKernelGGL(k_pick_check<11>, g, b, 0, s, c, nodes); break;
     default: return hipErrorInvalidValue;
   }
+  hipLaunchKernelGGL(k_pick_exact, dim3((c.pick.n_nodes + 63) / 64), dim3(64), 0, s, c.pick.n_nodes, c.n_shells + 3,
+                     nodes, c.pick.stride);
   return hipGetLastError();
 }
 
