@@ -56,9 +56,12 @@ __device__ __forceinline__ void count_outcome_words(const mcd_electron_rec* __re
 
 // ---------------------------------------------------------------------------
 // Electrons a wavefront goes on with in the window form once the work counter is
-// spent (one group of 4 lanes each).  Their last 1000 to 5000 steps cost 1.4 to
-// 1.9 us each with one lane per electron.  Launches of 2^20 electrons in us
-// without it and at 8 and 16: @@
+// spent: 16, the most that groups of 4 lanes hold.  Their last 1000 to 5000 steps
+// cost 1.4 to 1.9 us each with one lane per electron.  us without it, at 8 and at
+// 16: inline, 2^20 electrons, Cu 6090, 5520 and 5420, Au 14060, 11870 and 11530,
+// Al 8410, 7960 and 7860; continuous JL 4210, 4000 and 3980, explicit law 6510,
+// 6200 and 6270; served, 2^22 electrons, Cu 14750, 14280 and 14150, Au 34280,
+// 31390 and 30880.
 constexpr int kDrain = 16;
 
 // ---------------------------------------------------------------------------
@@ -378,8 +381,9 @@ static size_t svc_lds_bytes(const DevCfg& c, int block) {
 
 // Launches without scatter rows take a kernel without their tests in the step
 // (us with and without, 2^22 electrons: Cu, 7 channels 14451 and 14166, Al 6780
-// and 6633, Si 12988 and 12636).  From 9 channels on it spills more at 64 VGPRs
-// (Au, 11 channels 29703 and 33185), and the one with the tests serves both.
+// and 6633, Si 12988 and 12636; Au with 8 channels 20290 and 19910).  From 9
+// channels on it spills more at 64 VGPRs (9 channels 20720 and 21000, 10 21060 and
+// 21450, 11 21620 and 24070), and the one with the tests serves both.
 template <int NCH>
 constexpr bool kLean = NCH <= 8;
 
