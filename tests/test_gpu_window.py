@@ -1,6 +1,8 @@
 """Launches with several lanes per electron (mcd_window.hip) against one lane
 per electron: the same formulas step by step, so records, scatter rows and
-counters are equal bit for bit."""
+counters are equal bit for bit.  The inline kernel (guard="inline", an explicit
+block) begins with one lane per electron and gives several to the last 16 of a
+wavefront; test_gpu_window_reference.py compares with kernels that do not."""
 import numpy as np
 import pytest
 
@@ -17,7 +19,7 @@ def _transport(material="Cu", E0=20000.0, Emin=1000.0, Wc=50.0, tilt=70.0, **kw)
     return engine.Transport(material, E0, Emin, Wc=Wc, s_tilt=tilt, tol_E=1e-2, tol_W=1e-2, grid_search="library", **kw)
 
 
-# FP64 kernels and continuous mode have one form for an explicit block
+# one lane per electron: FP64 to the end, continuous mode but for the last 16 of a wavefront
 ONE_LANE = dict(block=256)
 FP64 = _abi.PREC_FP64
 
@@ -34,8 +36,8 @@ def cu():
     return _transport()
 
 
-# the counts around which the lanes per electron change (256 CUs: 3840 << 6 =
-# 7680 << 5 = .. = 98304 * 2.5), one electron, one short of and past a wavefront
+# counts around which the lanes per electron change (256 CUs: 3840 << 6 = 7680 << 5
+# = ..; one lane from 81921 on), one electron, one short of and past a wavefront
 @pytest.mark.parametrize("n", [1, 3, 63, 65, 3840, 3841, 7680, 7681, 15361, 30720, 30721, 98304, 98305])
 def test_ds_sizes_equal_one_lane_per_electron(cu, n):
     _same(cu.run(n, seed=n), cu.run(n, seed=n, guard="inline"))
@@ -88,7 +90,7 @@ def test_fp64_configurations_and_rows_equal_one_lane_per_electron(kw):
     _same(tr.run(40, **kw), tr.run(40, **kw, **ONE_LANE))
 
 
-# continuous mode: one wavefront per SIMD (65536 lanes), quads to two (explicit law: to one)
+# continuous mode: one wavefront per SIMD (65536 lanes), quads to three (explicit law: to one)
 @pytest.mark.parametrize("law", ["classical", "JL", "explicit"])
 @pytest.mark.parametrize("n", [1, 65, 1024, 1025, 8193, 16384, 16385, 32769])
 def test_continuous_sizes_equal_one_lane_per_electron(law, n):
@@ -111,7 +113,7 @@ def test_continuous_configurations_and_rows_equal_one_lane_per_electron(kw):
 
 
 # The last electrons of a large launch go on with several lanes each.  Forms
-# without that: wavefront budgets other than 4 per SIMD, the served guard.
+# without that: wavefront budgets other than 4 per SIMD.
 @pytest.mark.parametrize("kw", [
     dict(),
     dict(material="Au", E0=30000.0, Wc=20.0),
