@@ -1624,8 +1624,19 @@ extern "C" int mcd_backward(mcd_ctx* ctx, const mcd_config* cfg, const mcd_table
   const int per_cu = bwd_blocks_per_cu(c, A, jac, block);
   uint64_t want = (n + block - 1) / block;
   uint64_t grid = (uint64_t)ctx->n_cu * (uint64_t)per_cu;
+  const uint64_t lanes = grid * (uint64_t)block;
   if (grid > want) grid = want;
   if (grid < 1) grid = 1;
+  A.one_each = n <= grid * (uint64_t)block;
+  // Issue priorities shorten the end of a launch and cost 1 to 3 % of its steps:
+  // not with less than two wavefronts per SIMD, not for short replays (us without
+  // and with: Si 5 keV, 60 events by the model, JL 2^20 electrons 1301 and 1332),
+  // and in continuous mode not with more than 16 electrons per lane (Cu 20 keV, 309
+  // events, 2^18 1791 and 1587, 2^20 4392 and 4118, 2^22 13319 and 12934, 2^24
+  // 47377 and 47807; DS 2^20 9395 and 8349, 2^24 95097 and 94866).
+  const bool prio = work_per_electron(*cfg) >= 100. && n >= 128ull * 4 * (uint64_t)ctx->n_cu &&
+                    (cfg->mode == MCD_MODE_DS || n < 16 * lanes);
+  A.prio_mask = prio ? kBwdPrioSteps - 1 : ~0u;
   HIP_TRY(ctx, launch_fill_u64(ctx->d_queue, 0ull, 1, s));
   HIP_TRY(ctx, launch_backward(c, A, jac, (int)grid, block, s));
   return MCD_OK;

@@ -179,7 +179,13 @@ constexpr uint32_t kBwdStepCap = 1u << 22;
 // and the table descriptors are selected from LDS.  Cu 20 keV 70 deg on MI355X,
 // us: 1000 electrons 3245 to 2787, 2^18 5341 to 5008, 2^20 10481 to 9747, 2^22
 // 30116 to 27443.
-template <int MODE, int NCH, bool JAC>
+// Continuous mode's steps are short and its larger launches bound by issue, so it
+// has kernels of its own for launches with one electron per lane (ONE), the only
+// ones to read the upstream gradients unconditionally (us without and with: Cu 20
+// keV 65536 electrons 942 and 842, 2^24 47377 and 48955), and with and without
+// issue priorities (PRIO: the test at each step takes 0.8 %).  DS has one kernel
+// with the tests for both.
+template <int MODE, int NCH, bool JAC, bool ONE, bool PRIO>
 __global__ __launch_bounds__(256) void k_backward(DevCfg c, BwdArgs A) {
   extern __shared__ float lds[];
   float* nodes = lds;
@@ -219,7 +225,7 @@ __global__ __launch_bounds__(256) void k_backward(DevCfg c, BwdArgs A) {
   bool active = false, open = true;
   WaveQueue wq;
   // one electron per lane: the wavefront's only reservation is its own 64
-  const bool one_each = A.n <= (uint64_t)gridDim.x * blockDim.x;
+  const bool one_each = MODE == MCD_MODE_DS ? A.one_each != 0 : ONE;
   if (one_each) {
     wq.next = (uint64_t)blockIdx.x * blockDim.x + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
     wq.end = wq.next + 64;
@@ -231,7 +237,7 @@ __global__ __launch_bounds__(256) void k_backward(DevCfg c, BwdArgs A) {
   float dE[3], dz[3], dw[3], S[3];
   float dd[3][3], dy[3][3];  // [slot][component]; DS keeps slot 1 implicit (rigid tilt)
 
-  uint32_t iter = 0;
+  [[maybe_unused]] uint32_t iter = 0;
   while (true) {
     // key words as loop-carried SGPR values, set where all lanes are converged
     // (keeps the twenty round keys from being hoisted and spilled)
@@ -266,10 +272,9 @@ __global__ __launch_bounds__(256) void k_backward(DevCfg c, BwdArgs A) {
     }
     if (!__any(active)) break;
     // Wavefronts with high-energy electrons (the longest replays left) issue
-    // before the others on their SIMD, as in the served-guard kernel: 2^20
-    // electrons of Cu 20 keV in 8487 us instead of 9466, of Au 30 keV in 18901
-    // instead of 20792.
-    if ((iter++ & 7u) == 0u) {
+    // before the others on their SIMD, as in the served-guard kernel, in the
+    // launches that gain by it (see mcd_backward).
+    if (PRIO && (iter++ & A.prio_mask) == 0u) {
       const float span = c.E0_hi - Emin;
       if (__any(active && E > Emin + 0.5f * span)) __builtin_amdgcn_s_setprio(3);
       else if (__any(active && E > Emin + 0.2f * span)) __builtin_amdgcn_s_setprio(2);
@@ -366,6 +371,15 @@ __global__ __launch_bounds__(256) void k_backward(DevCfg c, BwdArgs A) {
             if (bp[i] >= 0) atomicAdd(&hist[4 * bp[i] + 1 + i], f);
             if (bm[i] >= 0) atomicAdd(&hist[4 * bm[i] + 1 + i], -f);
           }
+        }
+      } else if (MODE == MCD_MODE_CONT && !ONE) {
+        const float g = base ? gup[0] + gup[1 + b] : 0.f;
+        accv += C * g;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+          const float gp = bp[i] >= 0 ? gup[0] + gup[1 + bp[i]] : 0.f;
+          const float gm = bm[i] >= 0 ? gup[0] + gup[1 + bm[i]] : 0.f;
+          accg[i] += dC[i] * g + C * A.inv_2delta[i] * (gp - gm);
         }
       } else {
         // every lane reads (bin 0 for a dead side), so that the reads go out together
@@ -598,25 +612,33 @@ static size_t bwd_lds_bytes(const DevCfg& c, const BwdArgs& A, bool jac) {
   return sizeof(float) * (size_t)bwd_tab_offset(A, jac) + (c.mode == MCD_MODE_DS ? 2 * sizeof(DevTable) : 0);
 }
 
+template <bool JAC, bool PRIO>
+static const void* bwd_kernel_cont(const BwdArgs& A) {
+  return A.one_each ? reinterpret_cast<const void*>(&k_backward<MCD_MODE_CONT, 4, JAC, true, PRIO>)
+                    : reinterpret_cast<const void*>(&k_backward<MCD_MODE_CONT, 4, JAC, false, PRIO>);
+}
 template <bool JAC>
-static const void* bwd_kernel(const DevCfg& c) {
-  if (c.mode != MCD_MODE_DS) return reinterpret_cast<const void*>(&k_backward<MCD_MODE_CONT, 4, JAC>);
+static const void* bwd_kernel(const DevCfg& c, const BwdArgs& A) {
+  if (c.mode != MCD_MODE_DS)
+    return A.prio_mask == kBwdPrioSteps - 1 ? bwd_kernel_cont<JAC, true>(A) : bwd_kernel_cont<JAC, false>(A);
   switch (c.n_shells + 3) {
-    case 4: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 4, JAC>);
-    case 5: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 5, JAC>);
-    case 6: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 6, JAC>);
-    case 7: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 7, JAC>);
-    case 8: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 8, JAC>);
-    case 9: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 9, JAC>);
-    case 10: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 10, JAC>);
-    default: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 11, JAC>);
+    case 4: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 4, JAC, false, true>);
+    case 5: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 5, JAC, false, true>);
+    case 6: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 6, JAC, false, true>);
+    case 7: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 7, JAC, false, true>);
+    case 8: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 8, JAC, false, true>);
+    case 9: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 9, JAC, false, true>);
+    case 10: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 10, JAC, false, true>);
+    default: return reinterpret_cast<const void*>(&k_backward<MCD_MODE_DS, 11, JAC, false, true>);
   }
 }
-static const void* bwd_kernel(const DevCfg& c, bool jac) { return jac ? bwd_kernel<true>(c) : bwd_kernel<false>(c); }
+static const void* bwd_kernel(const DevCfg& c, const BwdArgs& A, bool jac) {
+  return jac ? bwd_kernel<true>(c, A) : bwd_kernel<false>(c, A);
+}
 
 int bwd_blocks_per_cu(const DevCfg& c, const BwdArgs& A, bool jac, int block) {
   int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, bwd_kernel(c, jac), block, bwd_lds_bytes(c, A, jac)) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, bwd_kernel(c, A, jac), block, bwd_lds_bytes(c, A, jac)) !=
       hipSuccess)
     return 1;
   return nb < 1 ? 1 : nb;
@@ -624,7 +646,7 @@ int bwd_blocks_per_cu(const DevCfg& c, const BwdArgs& A, bool jac, int block) {
 
 hipError_t launch_backward(const DevCfg& c, const BwdArgs& A, bool jac, int grid, int block, hipStream_t s) {
   void* args[] = {(void*)&c, (void*)&A};
-  return hipLaunchKernel(bwd_kernel(c, jac), dim3(grid), dim3(block), args, bwd_lds_bytes(c, A, jac), s);
+  return hipLaunchKernel(bwd_kernel(c, A, jac), dim3(grid), dim3(block), args, bwd_lds_bytes(c, A, jac), s);
 }
 
 }  // namespace mcd

@@ -88,7 +88,10 @@ struct BwdArgs {
   const float* m_score_e;      // DS: energy score of each Moller table column pick
   const float* g_score_e;      // DS: energy score of each Gryzinski table column pick
   float inv_wc, inv_nw1;       // DS: 1 / Wc, 1 / (nW_Moller - 1)
+  int one_each;                // the launch has a lane for every electron
+  uint32_t prio_mask;          // steps between issue priorities, less one (all ones: none)
 };
+constexpr uint32_t kBwdPrioSteps = 8;
 
 hipError_t launch_bwd_nodes(const DevCfg& c, int n_nodes, double lnE0, double dln, float* nodes, int stride,
                             hipStream_t s);

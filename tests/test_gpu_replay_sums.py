@@ -44,3 +44,28 @@ def test_repeated_products_are_equal_to_rounding(kw, n):
     for _ in range(6):
         b = sums(n)
         assert (np.abs(b - a) <= tol).all(), (b - a) / np.maximum(size, 1e-300)
+
+
+# The replay's forms on 256 CUs: issue priorities from 131072 electrons (not for
+# Si 5 keV), one electron per lane up to 327680 (DS) and 393216, none of both in
+# continuous mode from 16 electrons per lane.  Float32 sums of up to ~10^4 terms
+# per lane and bin: within 1e-4 of the sum of magnitudes.
+@pytest.mark.parametrize("n", [131071, 131072, 327680, 327681, 393216, 393217, 16 * 393216])
+@pytest.mark.parametrize("kw", [dict(material="Cu", Wc=50.0, tol_E=1e-2, tol_W=1e-2),
+                                dict(material="Au", mode="cont", bethe_model="JL"),
+                                dict(material="Si", mode="cont", bethe_model="classical")], ids=str)
+def test_products_equal_jacobians_in_every_form(kw, n):
+    import torch
+    if kw["material"] == "Cu" and n > 400000:
+        n = 400000
+    kw = dict(kw)
+    tr = engine.Transport(kw.pop("material"), 5000.0, 1000.0, s_tilt=60.0, **kw)
+    g = np.random.default_rng(2).standard_normal(65).astype(np.float32)
+    J, out = np.asarray(tr.jacobian(n, seed=5)), np.asarray(tr.vjp(n, torch.from_numpy(g), seed=5))
+    assert J[0, 0] > 0 and np.isfinite(J).all()
+    want, size = g.astype(np.float64) @ J, np.abs(g).astype(np.float64) @ np.abs(J)
+    assert (np.abs(out - want) <= 1e-4 * np.maximum(size, np.abs(J).sum() * 1e-3)).all()
+    # the same electrons in two launches
+    h = n // 2
+    halves = (np.asarray(tr.jacobian(h, seed=5)) * h + np.asarray(tr.jacobian(n - h, seed=5, first=h)) * (n - h)) / n
+    assert (np.abs(halves - J) <= 1e-4 * np.maximum(np.abs(J), np.abs(J).sum() * 1e-3)).all()
