@@ -25,8 +25,8 @@
 //      in three lanes of a quad.  Steps past the electron's end are dropped.
 // Every formula is the one of transport_loop and k_transport_f64, so records,
 // scatter rows and counters are the same bit for bit.
-// Cycles of a 64-lane window (Cu 20 keV, FP32): random words 660, energy chain
-// 9900, geometry 14100 (220 a step), the rest 1150; 64 steps of one lane on its
+// Cycles of a 64-lane window (Cu 20 keV, FP32; clock readings in a copy of the
+// kernel, a few electrons): random words 660, energy chain 9900, geometry 14100 (220 a step), the rest 1150; 64 steps of one lane on its
 // own take 160000.
 #pragma once
 
